@@ -262,9 +262,11 @@ int tgohip_linear(tgohip_ctx* ctx, int handle, const void* x, int x_dtype, int M
  * two contexts at once) race; calls in stream order do not. */
 int tgohip_linear_noalloc(tgohip_ctx* ctx, int handle, const void* x, int x_dtype, int M,
                           void* y, int y_dtype);
-/* Bytes of split-K partials a linear call over M rows of a handle's weight
- * with activations of x_dtype (TGOHIP_F16, TGOHIP_F32 or TGOHIP_F16X2) needs:
- * 0 when it runs unsplit. tgohip_linear_noalloc refuses calls above 64 MiB. */
+/* The split-K bytes by which tgohip_linear_noalloc takes or refuses a call over
+ * M rows of a handle's weight with activations of x_dtype (TGOHIP_F16,
+ * TGOHIP_F32 or TGOHIP_F16X2): it refuses calls above 64 MiB. What a call
+ * writes there is at most this, or fits the array (few rows; f32 rows, which
+ * may go in bands, with the same result). */
 int tgohip_linear_workspace(tgohip_ctx* ctx, int handle, int x_dtype, int M, size_t* bytes);
 
 /* Dequantizes a handle's weight to f32 [K,N] on the device exactly as the

@@ -12,7 +12,7 @@ OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libtgohip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-HIP_SOURCES = ["runtime.hip", "kernels/attention.hip", "kernels/gemm.hip",
+HIP_SOURCES = ["runtime.hip", "kernels/attention.hip", "kernels/gemm.hip", "kernels/gemm_rows.hip",
                "kernels/elementwise.hip", "kernels/probe.hip"]
 CXX_SOURCES = ["host/hostlogic.cpp", "host/checkpoint.cpp"]
 

@@ -116,10 +116,15 @@ size_t packed_scale_halves(int form, int K, int N);
 int repack_enqueue(int form, const void* plane, const uint16_t* scales, const uint16_t* zeros,
                    int K, int N, PackedWeight& w, int nb_stride, int nb_off, hipStream_t st);
 int dequant_enqueue(const PackedWeight& w, void* out, bool f16out, hipStream_t st);
-// Split-K workspace of a call: xk < 0 bounds every activation type and
-// epilogue; an XK_* value gives exactly what an f32/f16-epilogue call over
-// that activation type uses.
-size_t gemm_workspace_bytes(const PackedWeight& w, int M, int ncu, int xk = -1);
+// The most split-K workspace a call over M rows uses.
+size_t gemm_workspace_bytes(const PackedWeight& w, int M, int ncu);
+// The split-K bytes by which linear_noalloc takes or refuses a call over
+// activations of kind xk with an f32 or f16 epilogue.
+size_t gemm_limit_bytes(const PackedWeight& w, int M, int ncu, int xk);
+// Workspace bytes for a call over f32 activations that are split into a pair
+// first (0: the call splits them as it reads them). A smaller workspace makes
+// the call go in bands of rows, with the same sums.
+size_t gemm_f32_workspace_bytes(const PackedWeight& w, int M, int ncu);
 // With defer != nullptr a split-K launch leaves its partial planes in the
 // workspace ([splits][M][N] f32) and sets *defer = splits instead of running
 // the reduction; the caller folds them into the consumer (rmsnorm,

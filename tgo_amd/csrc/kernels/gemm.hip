@@ -15,8 +15,16 @@
 //   int8: two u32 per substep; bytes hold k offsets 0,2,1,3 as q+128 so the
 //         0x00FF00FF mask yields consecutive-k f16 pairs (1024+b).
 //   f16:  eight halves per substep.
+// A load takes 16 bytes per lane, the 64 lanes' side by side: 1 KiB of whole
+// cache lines (int8: substeps 0-1, then 2-3; f16: one substep). With a lane's
+// own 32 (int8) or 64 (f16) bytes side by side instead, each load touched every
+// line of the burst: gemm_rows_kernel over [4096, 24576] of f16 weights at one
+// row took 61.9 us (3.3 TB/s) against 32.1 (6.3 TB/s).
 // Dequantized value: round-to-nearest-even f16 of the exact (q - z) * s, which
 // is computed with one exact packed subtraction and one rounded packed multiply.
+//
+// Few rows, and small weights, run gemm_rows_kernel (gemm_rows.hip) or
+// gemm_gemv_kernel; the rest of this comment is the tiled kernels.
 //
 // Tiling: waves side by side in N, each MW x 64 (MW/32 x 2 MFMA blocks of
 // 32x32); a workgroup of 4 waves owns MW rows x 256 columns (gemm_pipe_kernel
@@ -27,319 +35,13 @@
 // the product keeps ~22 bits of the activation. Split-K over grid.z writes f32
 // partials that a reduction kernel (or the consumer) sums in split order
 // (deterministic).
-#include "../common.h"
+#include "gemm_weights.h"
 
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
 namespace tgohip {
-
-struct GemmArgs {
-  const void* x;        // [M,K] f16 or f32 (or the hi plane of an XK_X2 pair)
-  const void* xlo;      // XK_X2: the lo plane [M,K] f16; null otherwise
-  const void* wp;       // packed payload
-  const half_t* ws;     // packed scales (form dependent)
-  const half_t* wz;     // packed zero+1024 (I4_TGO only)
-  void* y;              // output (EPI dependent)
-  float* part;          // split-K partials: split s at part + s * pstride, [M][N]
-  size_t pstride;
-  int M, K, N;
-  int ksteps_per_split;
-};
-
-__device__ __forceinline__ half2_t as_h2(uint32_t u) {
-  union { uint32_t u; half2_t h; } c;
-  c.u = u;
-  return c.h;
-}
-
-// ---- dequantization of one substep's B fragment (8 consecutive k) ----------
-__device__ __forceinline__ half8_t deq_i4_sym(uint32_t w, half_t s) {
-  const half2_t sp = {s, s};
-  // A nibble in bits 0-3 of a 16-bit half merged into 0x6400 (1024.0) reads
-  // as 1024 + q; one in bits 4-7 merged into 0x5400 (64.0, whose mantissa bit
-  // 4 is worth 1) reads as 64 + q. Subtracting 1032 or 72 leaves q - 8
-  // exactly, so substeps 0/1 come from w and 2/3 from w >> 8 with one shift.
-  // The masks sit in registers so each mask-and-merge is one v_and_or_b32
-  // (its encoding takes no literal constants).
-  uint32_t m0 = 0x000F000Fu, m1 = 0x00F000F0u, g0 = 0x64006400u, g1 = 0x54005400u;
-  asm("" : "+v"(m0), "+v"(m1), "+v"(g0), "+v"(g1));
-  const half2_t b0 = {(half_t)1032.f, (half_t)1032.f}, b1 = {(half_t)72.f, (half_t)72.f};
-  const uint32_t w8 = w >> 8;
-  const half2_t h[4] = {(as_h2((w & m0) | g0) - b0) * sp, (as_h2((w & m1) | g1) - b1) * sp,
-                        (as_h2((w8 & m0) | g0) - b0) * sp, (as_h2((w8 & m1) | g1) - b1) * sp};
-  half8_t o;
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    o[2 * j] = h[j][0];
-    o[2 * j + 1] = h[j][1];
-  }
-  return o;
-}
-// The codes q - 8 of one substep's B fragment, unscaled: small integers, exact
-// in f16 (the masks and merge constants of deq_i4_sym).
-__device__ __forceinline__ half8_t i4_sym_codes(uint32_t w) {
-  uint32_t m0 = 0x000F000Fu, m1 = 0x00F000F0u, g0 = 0x64006400u, g1 = 0x54005400u;
-  asm("" : "+v"(m0), "+v"(m1), "+v"(g0), "+v"(g1));
-  const half2_t b0 = {(half_t)1032.f, (half_t)1032.f}, b1 = {(half_t)72.f, (half_t)72.f};
-  const uint32_t w8 = w >> 8;
-  const half2_t h[4] = {as_h2((w & m0) | g0) - b0, as_h2((w & m1) | g1) - b1,
-                        as_h2((w8 & m0) | g0) - b0, as_h2((w8 & m1) | g1) - b1};
-  half8_t o;
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    o[2 * j] = h[j][0];
-    o[2 * j + 1] = h[j][1];
-  }
-  return o;
-}
-__device__ __forceinline__ half8_t deq_i4_asym(uint32_t w, half8_t s, half8_t zz) {
-  half8_t o;
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    half2_t h = as_h2(((w >> (4 * j)) & 0x000F000Fu) | 0x64006400u);
-    const half2_t z2 = {zz[2 * j], zz[2 * j + 1]};
-    const half2_t s2 = {s[2 * j], s[2 * j + 1]};
-    h = h - z2;
-    h = h * s2;
-    o[2 * j] = h[0];
-    o[2 * j + 1] = h[1];
-  }
-  return o;
-}
-__device__ __forceinline__ half8_t deq_i8(uint32_t w0, uint32_t w1, half8_t s) {
-  const half2_t bias = {(half_t)1152.f, (half_t)1152.f};
-  half8_t o;
-  const uint32_t ws[2] = {w0, w1};
-#pragma unroll
-  for (int u = 0; u < 2; u++) {
-    half2_t lo = as_h2((ws[u] & 0x00FF00FFu) | 0x64006400u);
-    half2_t hi = as_h2(((ws[u] >> 8) & 0x00FF00FFu) | 0x64006400u);
-    const half2_t s0 = {s[4 * u], s[4 * u + 1]}, s1 = {s[4 * u + 2], s[4 * u + 3]};
-    lo = (lo - bias) * s0;
-    hi = (hi - bias) * s1;
-    o[4 * u] = lo[0];
-    o[4 * u + 1] = lo[1];
-    o[4 * u + 2] = hi[0];
-    o[4 * u + 3] = hi[1];
-  }
-  return o;
-}
-
-// The lane's raw material for one (nb, ks): payload plus the scales it needs,
-// sized per form so no register is spent on another form's fields.
-template <int FORM> struct BRaw;
-template <> struct BRaw<TGOHIP_FORM_F16> { uint4 p[4]; };
-template <> struct BRaw<TGOHIP_FORM_I8> { uint4 p[2]; uint4 s[4]; };
-template <> struct BRaw<TGOHIP_FORM_I4_TGO> { uint4 p; uint4 s[4]; uint4 z[4]; };
-template <> struct BRaw<TGOHIP_FORM_I4_SYM> { uint4 p; uint32_t s; };
-
-typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-
-// A 16-byte weight load; NT: non-temporal (the nt bit), for a launch that
-// reads each weight once. The small-M kernel's int4 gate/up at one row went
-// from 15.6 to 13.5 us with it, the LM head from 70.7 to 64.8; the pipelined
-// kernel's row tiles share weights through L2, and nt loads made its 64- and
-// 128-row down 12-18% slower.
-template <bool NT>
-__device__ __forceinline__ uint4 ldw16(const void* p) {
-  if constexpr (NT) {
-    const u32x4_t v = __builtin_nontemporal_load((const u32x4_t*)p);
-    return make_uint4(v.x, v.y, v.z, v.w);
-  } else {
-    return *(const uint4*)p;
-  }
-}
-
-template <bool NT = false>
-__device__ __forceinline__ void load_braw(const GemmArgs& g, int nb, int ks, int lane,
-                                          BRaw<TGOHIP_FORM_F16>& r) {
-  const size_t slot = ((size_t)nb * (g.K / 64) + ks) * 64 + lane;
-  const uint4* pp = (const uint4*)((const char*)g.wp + slot * 64);
-#pragma unroll
-  for (int i = 0; i < 4; i++) r.p[i] = ldw16<NT>(pp + i);
-}
-template <bool NT = false>
-__device__ __forceinline__ void load_braw(const GemmArgs& g, int nb, int ks, int lane,
-                                          BRaw<TGOHIP_FORM_I8>& r) {
-  const int KS = g.K / 64;
-  const size_t slot = ((size_t)nb * KS + ks) * 64 + lane;
-  const uint4* pp = (const uint4*)((const char*)g.wp + slot * 32);
-  r.p[0] = ldw16<NT>(pp);
-  r.p[1] = ldw16<NT>(pp + 1);
-  const int h = lane >> 5;
-#pragma unroll
-  for (int j = 0; j < 4; j++) r.s[j] = *(const uint4*)(g.ws + ((((size_t)nb * KS + ks) * 4 + j) * 2 + h) * 8);
-}
-template <bool NT = false>
-__device__ __forceinline__ void load_braw(const GemmArgs& g, int nb, int ks, int lane,
-                                          BRaw<TGOHIP_FORM_I4_TGO>& r) {
-  const int KS = g.K / 64;
-  const size_t slot = ((size_t)nb * KS + ks) * 64 + lane;
-  r.p = ldw16<NT>((const char*)g.wp + slot * 16);
-  const int h = lane >> 5;
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const size_t o = ((((size_t)nb * KS + ks) * 4 + j) * 2 + h) * 8;
-    r.s[j] = *(const uint4*)(g.ws + o);
-    r.z[j] = *(const uint4*)(g.wz + o);
-  }
-}
-template <bool NT = false>
-__device__ __forceinline__ void load_braw(const GemmArgs& g, int nb, int ks, int lane,
-                                          BRaw<TGOHIP_FORM_I4_SYM>& r) {
-  // (nb, ks) is uniform across the wave: a scalar base plus a 32-bit lane
-  // offset, so the loads need no 64-bit vector address arithmetic.
-  const size_t blk = (size_t)nb * (g.K / 64) + ks;
-  r.p = ldw16<NT>((const char*)g.wp + blk * 1024 + (uint32_t)lane * 16u);
-  r.s = *(const uint32_t*)((const char*)g.ws + blk * 128 + (uint32_t)(lane & 31) * 4u);
-}
-
-__device__ __forceinline__ uint32_t word_of(const uint4& p, int j) {
-  return j == 0 ? p.x : j == 1 ? p.y : j == 2 ? p.z : p.w;
-}
-
-union U16B { uint4 u; half8_t h; };
-
-__device__ __forceinline__ half8_t bfrag(const BRaw<TGOHIP_FORM_F16>& r, int j) {
-  U16B c;
-  c.u = r.p[j];
-  return c.h;
-}
-__device__ __forceinline__ half8_t bfrag(const BRaw<TGOHIP_FORM_I4_SYM>& r, int j) {
-  union { uint32_t u; half2_t h; } sc;
-  sc.u = r.s;
-  return deq_i4_sym(word_of(r.p, j), j < 2 ? sc.h[0] : sc.h[1]);
-}
-__device__ __forceinline__ half8_t bfrag(const BRaw<TGOHIP_FORM_I4_TGO>& r, int j) {
-  U16B s, z;
-  s.u = r.s[j];
-  z.u = r.z[j];
-  return deq_i4_asym(word_of(r.p, j), s.h, z.h);
-}
-__device__ __forceinline__ half8_t bfrag(const BRaw<TGOHIP_FORM_I8>& r, int j) {
-  const uint4 q = r.p[j >> 1];
-  const uint32_t w0 = (j & 1) ? q.z : q.x, w1 = (j & 1) ? q.w : q.y;
-  U16B s;
-  s.u = r.s[j];
-  return deq_i8(w0, w1, s.h);
-}
-
-// ---- exact dequantized weights as two f16 fragments ------------------------
-// hi = RNE_f16((q - z) * s) and lo = (q - z) * s - hi, each f16, so hi + lo is
-// the exact product tgo's CPU path multiplies (the f32 dequantization): (q - z)
-// has at most 8 significant bits and s 11, so the residual after hi's 11 bits
-// fits lo's (down to f16's subnormal spacing, 2^-24). lo comes from one fused
-// multiply-add, q*s - hi, rounded once and exact. An MFMA with each half gives
-// the product against the unrounded weight.
-__device__ __forceinline__ void split_pair(half2_t d, half2_t s2, half2_t& hi, half2_t& lo) {
-  hi = d * s2;
-  lo = __builtin_elementwise_fma(d, s2, -hi);
-}
-__device__ __forceinline__ void pack_pair(half8_t& o, int j, half2_t h) {
-  o[2 * j] = h[0];
-  o[2 * j + 1] = h[1];
-}
-template <int FORM>
-__device__ __forceinline__ void bfrag_split(const BRaw<FORM>& r, int j, half8_t& hi, half8_t& lo);
-template <>
-__device__ __forceinline__ void bfrag_split(const BRaw<TGOHIP_FORM_I4_SYM>& r, int j, half8_t& hi,
-                                            half8_t& lo) {
-  union { uint32_t u; half2_t h; } sc;
-  sc.u = r.s;
-  const half_t s = j < 2 ? sc.h[0] : sc.h[1];
-  const half2_t sp = {s, s};
-  const uint32_t w = word_of(r.p, j), w8 = w >> 8;
-  const half2_t b0 = {(half_t)1032.f, (half_t)1032.f}, b1 = {(half_t)72.f, (half_t)72.f};
-  // q - 8 exactly, as in deq_i4_sym (masks in registers: one v_and_or_b32 each)
-  uint32_t m0 = 0x000F000Fu, m1 = 0x00F000F0u, g0 = 0x64006400u, g1 = 0x54005400u;
-  asm("" : "+v"(m0), "+v"(m1), "+v"(g0), "+v"(g1));
-  const half2_t d[4] = {as_h2((w & m0) | g0) - b0, as_h2((w & m1) | g1) - b1,
-                        as_h2((w8 & m0) | g0) - b0, as_h2((w8 & m1) | g1) - b1};
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    half2_t h, l;
-    split_pair(d[i], sp, h, l);
-    pack_pair(hi, i, h);
-    pack_pair(lo, i, l);
-  }
-}
-template <>
-__device__ __forceinline__ void bfrag_split(const BRaw<TGOHIP_FORM_I4_TGO>& r, int j, half8_t& hi,
-                                            half8_t& lo) {
-  U16B s, z;
-  s.u = r.s[j];
-  z.u = r.z[j];
-  const uint32_t w = word_of(r.p, j);
-  uint32_t m0 = 0x000F000Fu, g0 = 0x64006400u;
-  asm("" : "+v"(m0), "+v"(g0));
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    // (1024 + q) - (1024 + z) = q - z exactly
-    const half2_t d = as_h2(((w >> (4 * i)) & m0) | g0) - half2_t{z.h[2 * i], z.h[2 * i + 1]};
-    half2_t h, l;
-    split_pair(d, half2_t{s.h[2 * i], s.h[2 * i + 1]}, h, l);
-    pack_pair(hi, i, h);
-    pack_pair(lo, i, l);
-  }
-}
-template <>
-__device__ __forceinline__ void bfrag_split(const BRaw<TGOHIP_FORM_I8>& r, int j, half8_t& hi,
-                                            half8_t& lo) {
-  const uint4 q = r.p[j >> 1];
-  const uint32_t ws[2] = {(j & 1) ? q.z : q.x, (j & 1) ? q.w : q.y};
-  U16B s;
-  s.u = r.s[j];
-  const half2_t bias = {(half_t)1152.f, (half_t)1152.f};
-  uint32_t m0 = 0x00FF00FFu, g0 = 0x64006400u;
-  asm("" : "+v"(m0), "+v"(g0));
-#pragma unroll
-  for (int u = 0; u < 2; u++) {
-    // (1024 + q + 128) - 1152 = q exactly
-    const half2_t dl = as_h2((ws[u] & m0) | g0) - bias;
-    const half2_t dh = as_h2(((ws[u] >> 8) & m0) | g0) - bias;
-    half2_t h, l;
-    split_pair(dl, half2_t{s.h[4 * u], s.h[4 * u + 1]}, h, l);
-    pack_pair(hi, 2 * u, h);
-    pack_pair(lo, 2 * u, l);
-    split_pair(dh, half2_t{s.h[4 * u + 2], s.h[4 * u + 3]}, h, l);
-    pack_pair(hi, 2 * u + 1, h);
-    pack_pair(lo, 2 * u + 1, l);
-  }
-}
-template <>
-__device__ __forceinline__ void bfrag_split(const BRaw<TGOHIP_FORM_F16>& r, int j, half8_t& hi,
-                                            half8_t& lo) {
-  hi = bfrag(r, j);  // f16 weights are exact as stored
-  lo = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-}
-
-// silu(g) = g / (1 + e^-g) (nn/blocks.go:62-66) with the hardware reciprocal
-// (v_rcp_f32, 1 ulp) in place of the IEEE division's ten-instruction sequence:
-// the SwiGLU epilogue of the C4 gate/up 209 -> 205 us.
-__device__ __forceinline__ float silu_f(float g) { return g * __builtin_amdgcn_rcpf(1.f + __expf(-g)); }
-
-// 16-byte slot of (row, k-chunk) in an LDS activation tile of 8 chunks per row.
-// The XOR with (row/2) % 8 spreads any 16 consecutive rows of one k-chunk over
-// all 64 banks (a bank row is 256 bytes = two tile rows), so the MFMA operand
-// reads (16 lanes = 16 rows per LDS cycle) and the row-wise stores are
-// conflict-free.
-__device__ __forceinline__ int a_slot(int row, int kc) { return row * 8 + (kc ^ ((row >> 1) & 7)); }
-
-// One SwiGLU output at element o of [M, N/2]: f16, f32, or the f16 hi plane
-// and the lo plane (f16(v - hi)) M*N/2 elements after it (the activation pair
-// the exact down projection reads).
-template <int EPI>
-__device__ __forceinline__ void store_swiglu(const GemmArgs& g, size_t o, float v) {
-  if (EPI == EPI_SWIGLU_F32) {
-    ((float*)g.y)[o] = v;
-  } else {
-    const half_t h = (half_t)v;
-    ((half_t*)g.y)[o] = h;
-    if (EPI == EPI_SWIGLU_X2) ((half_t*)g.y)[(size_t)g.M * (g.N / 2) + o] = (half_t)(v - (float)h);
-  }
-}
 
 // Epilogue shared by the GEMM kernels. Lane holds D[8*(r/4) + 4*h + (r%4)][c32]
 // of each 32x32 block; a split-K launch writes f32 partials for its split.
@@ -377,14 +79,6 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const float16_t
       }
     }
   }
-}
-
-// A workgroup barrier that orders LDS only: global loads in flight stay in
-// flight across it (__syncthreads would wait for them).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // ASPLIT (f32 activations, tgo's arithmetic): the activation is carried as f16
@@ -531,13 +225,38 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs g) {
 // block, so they travel by LDS DMA with the activation tile instead of in
 // registers (8 scale/zero pairs per lane per substep would not fit).
 template <int FORM> struct PipeB;
+template <> struct PipeB<TGOHIP_FORM_F16> { uint4 p[4]; };
 template <> struct PipeB<TGOHIP_FORM_I4_SYM> { uint4 p; uint32_t s; };
 template <> struct PipeB<TGOHIP_FORM_I4_TGO> { uint4 p; };
 template <> struct PipeB<TGOHIP_FORM_I8> { uint4 p[2]; };
 
-template <int FORM> constexpr bool pipe_lds_scales() { return FORM != TGOHIP_FORM_I4_SYM; }
+template <int FORM> constexpr bool pipe_lds_scales() {
+  return FORM == TGOHIP_FORM_I8 || FORM == TGOHIP_FORM_I4_TGO;
+}
 // Vector memory instructions a wave issues per k-step for its two B blocks.
-template <int FORM> constexpr int pipe_b_loads() { return FORM == TGOHIP_FORM_I4_TGO ? 2 : 4; }
+template <int FORM> constexpr int pipe_b_loads() {
+  return FORM == TGOHIP_FORM_F16 ? 8 : FORM == TGOHIP_FORM_I4_TGO ? 2 : 4;
+}
+// k-steps ahead that B is loaded: two for f16 weights, whose two blocks take
+// 32 registers per k-step.
+template <int FORM> constexpr int pipe_b_ahead() { return FORM == TGOHIP_FORM_F16 ? 2 : 3; }
+
+__device__ __forceinline__ void load_pipeb(const GemmArgs& g, int nb, int ks, int lane,
+                                           PipeB<TGOHIP_FORM_F16>& r) {
+  BRaw<TGOHIP_FORM_F16> b;
+  load_braw(g, nb, ks, lane, b);
+#pragma unroll
+  for (int i = 0; i < 4; i++) r.p[i] = b.p[i];
+}
+__device__ __forceinline__ half8_t pipe_bfrag(const PipeB<TGOHIP_FORM_F16>& r, int j, const half_t*, int, int) {
+  U16B c;
+  c.u = r.p[j];
+  return c.h;
+}
+__device__ __forceinline__ void pipe_bfrag_x(const PipeB<TGOHIP_FORM_F16>& r, int j, const half_t* sz, int b, int h,
+                                             half8_t& hi, half8_t&) {
+  hi = pipe_bfrag(r, j, sz, b, h);  // exact as stored: no lo part
+}
 
 __device__ __forceinline__ void load_pipeb(const GemmArgs& g, int nb, int ks, int lane,
                                            PipeB<TGOHIP_FORM_I4_SYM>& r) {
@@ -554,9 +273,9 @@ __device__ __forceinline__ void load_pipeb(const GemmArgs& g, int nb, int ks, in
 __device__ __forceinline__ void load_pipeb(const GemmArgs& g, int nb, int ks, int lane,
                                            PipeB<TGOHIP_FORM_I8>& r) {
   const size_t blk = (size_t)nb * (g.K / 64) + ks;
-  const uint4* pp = (const uint4*)((const char*)g.wp + blk * 2048 + (uint32_t)lane * 32u);
-  r.p[0] = pp[0];
-  r.p[1] = pp[1];
+  const char* pp = (const char*)g.wp + blk * 2048 + (uint32_t)lane * 16u;
+  r.p[0] = *(const uint4*)pp;
+  r.p[1] = *(const uint4*)(pp + 1024);
 }
 // Substep j's B fragment. sz: this wave's scale region of the k-step's stage
 // (scales of block b at b*64 + (2j + h)*8, zeros 128 halves further).
@@ -628,7 +347,11 @@ __device__ __forceinline__ void pipe_bfrag_x(const PipeB<TGOHIP_FORM_I8>& r, int
 // product x_hi q, x_lo q is exact and s_g multiplies in f32, so this is
 // tgo's f32 dequantize-then-dot up to f32 rounding order, with the lo.lo term
 // (2^-22 relative) dropped as in the three-MFMA form.
-template <int FORM, int EPI, int MW, int NW, int KQ = 1, bool EX = false>
+// TAIL: K may leave one to three k-steps after its groups of four. The tail
+// costs the factored kernel 1% at [4096, 24576] over 1152 rows (394-397 us
+// without, 399-401 with: its registers go from 238 to 256), so that kernel is
+// built both ways; the others are as fast with it.
+template <int FORM, int EPI, int MW, int NW, int KQ = 1, bool EX = false, bool TAIL = true>
 __global__ __launch_bounds__((64 * NW * KQ), (8 / (NW * KQ))) void gemm_pipe_kernel(
     GemmArgs g, int tiles_n, int tiles, int colmajor, int xsplit, QKRopeArgs qa) {
   constexpr int MB = MW / 32;
@@ -693,8 +416,8 @@ __global__ __launch_bounds__((64 * NW * KQ), (8 / (NW * KQ))) void gemm_pipe_ker
   const int nbw0 = tn * 2 * NW + wave * 2;
   const int m0 = tm * MW;
   const int KS = g.K / 64;
-  // k group q takes the q-th 1/KQ of the workgroup's k-steps (the host makes
-  // each a multiple of 4)
+  // k group q takes the q-th 1/KQ of the workgroup's k-steps (with KQ = 2 the
+  // host makes each a multiple of 4)
   const int nkw = min(KS, split * g.ksteps_per_split + g.ksteps_per_split) - split * g.ksteps_per_split;
   const int nk = nkw / KQ;
   const int ks0 = split * g.ksteps_per_split + kq * nk;
@@ -785,13 +508,14 @@ __global__ __launch_bounds__((64 * NW * KQ), (8 / (NW * KQ))) void gemm_pipe_ker
       else bh[b] = pipe_bfrag(bb[b], j, sz, b, h);
     }
   };
-  if (nk > 0) {  // nk is then a multiple of 4 (the host guarantees it)
+  if (nk > 0) {
 #pragma unroll
     for (int b = 0; b < 2; b++) load_pipeb(g, nbl[b], kpos(0), lane, bq[0][b]);
 #pragma unroll
     for (int b = 0; b < 2; b++) load_pipeb(g, nbl[b], kpos(1), lane, bq[1][b]);
 #pragma unroll
-    for (int b = 0; b < 2; b++) load_pipeb(g, nbl[b], kpos(2), lane, bq[2][b]);
+    for (int b = 0; b < 2; b++)
+      if (pipe_b_ahead<FORM>() == 3) load_pipeb(g, nbl[b], kpos(2), lane, bq[2][b]);
     PIPE_DMA_A(kpos(0), 0);
     PIPE_DMA_A(kpos(1), 1);
     PIPE_DMA_A(kpos(2), 2);
@@ -802,166 +526,200 @@ __global__ __launch_bounds__((64 * NW * KQ), (8 / (NW * KQ))) void gemm_pipe_ker
     read_a((const half8_t*)(As[0] + aq), h, afc, afcl);
     read_b(bq[0], 0, Sz[0] + sq + wave * 256, bfc, bfcl);
   }
-  for (int kk = 0; kk < nk; kk += 4) {
+  auto step = [&](auto uc, int kk) {
+    constexpr int u = decltype(uc)::value;
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
+    for (int b = 0; b < 2; b++)
+      load_pipeb(g, nbl[b], kpos(kk + u + pipe_b_ahead<FORM>()), lane, bq[(u + pipe_b_ahead<FORM>()) % 4][b]);
+    // Keep the loads issued here, ahead of the MFMAs: the scheduler would
+    // otherwise sink them next to their use and expose their latency.
+    __builtin_amdgcn_sched_barrier(0);
+    // Raised wave priority through the MFMA phase: of the two waves sharing
+    // a SIMD, the one issuing MFMAs goes first.
+    __builtin_amdgcn_s_setprio(1);
+    const half8_t* A = (const half8_t*)(As[u] + aq);
+    const half8_t* An = (const half8_t*)(As[(u + 1) % 4] + aq);
+    // Substep j's MFMAs run while the next substep's A fragments are read
+    // from LDS and its B fragments dequantized; the group barriers
+    // interleave them (1 MFMA, 1 LDS read, 5 VALU) so the matrix core stays
+    // fed.
 #pragma unroll
-      for (int b = 0; b < 2; b++) load_pipeb(g, nbl[b], kpos(kk + u + 3), lane, bq[(u + 3) % 4][b]);
-      // Keep the loads issued here, ahead of the MFMAs: the scheduler would
-      // otherwise sink them next to their use and expose their latency.
-      __builtin_amdgcn_sched_barrier(0);
-      // Raised wave priority through the MFMA phase: of the two waves sharing
-      // a SIMD, the one issuing MFMAs goes first.
-      __builtin_amdgcn_s_setprio(1);
-      const half8_t* A = (const half8_t*)(As[u] + aq);
-      const half8_t* An = (const half8_t*)(As[(u + 1) % 4] + aq);
-      // Substep j's MFMAs run while the next substep's A fragments are read
-      // from LDS and its B fragments dequantized; the group barriers
-      // interleave them (1 MFMA, 1 LDS read, 5 VALU) so the matrix core stays
-      // fed.
+    for (int j = 0; j < 4; j++) {
+      half8_t afn[MB], bfn[2], afnl[MB], bfnl[2];
+      if (j < 3) {
+        read_a(A, 2 * (j + 1) + h, afn, afnl);
+        read_b(bq[u], j + 1, Sz[u] + sq + wave * 256, bfn, bfnl);
+      } else {
+        read_a(An, h, afn, afnl);
+        read_b(bq[(u + 1) % 4], 0, Sz[(u + 1) % 4] + sq + wave * 256, bfn, bfnl);
+      }
+      if constexpr (FX) {
+        // substeps 0-1 are the k-step's first scale group, 2-3 its second;
+        // an even substep starts the group's sums, an odd one ends them
+        // and scales them into acc
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        half8_t afn[MB], bfn[2], afnl[MB], bfnl[2];
-        if (j < 3) {
-          read_a(A, 2 * (j + 1) + h, afn, afnl);
-          read_b(bq[u], j + 1, Sz[u] + sq + wave * 256, bfn, bfnl);
-        } else {
-          read_a(An, h, afn, afnl);
-          read_b(bq[(u + 1) % 4], 0, Sz[(u + 1) % 4] + sq + wave * 256, bfn, bfnl);
-        }
-        if constexpr (FX) {
-          // substeps 0-1 are the k-step's first scale group, 2-3 its second;
-          // an even substep starts the group's sums, an odd one ends them
-          // and scales them into acc
+        for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-          for (int mb = 0; mb < MB; mb++)
+          for (int b = 0; b < 2; b++)
+            accg[mb][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                afc[mb], bfc[b], (j & 1) ? accg[mb][b] : zero16, 0, 0, 0);
 #pragma unroll
-            for (int b = 0; b < 2; b++)
-              accg[mb][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                  afc[mb], bfc[b], (j & 1) ? accg[mb][b] : zero16, 0, 0, 0);
+        for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-          for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-            for (int b = 0; b < 2; b++)
-              accg[mb][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afcl[mb], bfc[b], accg[mb][b], 0, 0, 0);
-          if (j & 1) {
-            // The scaling reads the group's last MFMAs, so this wave has no
-            // MFMA to issue beside it: at the lower priority the other wave
-            // on the SIMD issues first (the C4 step 40.1-40.5 -> 39.1 ms;
-            // gate/up 407 -> 390-399 us, QKV 116 -> 106-111 us). With two k
-            // groups per workgroup the isolated block spilled more (18
-            // VGPRs, not 8-11), so they keep the interleave below. The
-            // lane's column scale of this group: bq[u] holds step u's two
-            // per lane column.
-            if constexpr (KQ == 1) {
-              __builtin_amdgcn_sched_barrier(0);
-              __builtin_amdgcn_s_setprio(0);
-            }
-#pragma unroll
-            for (int b = 0; b < 2; b++) {
-              union { uint32_t u; half2_t h; } sc;
-              sc.u = bq[u][b].s;
-              const float s = (float)sc.h[j >> 1];
-#pragma unroll
-              for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) acc[mb][b][r] = __builtin_fmaf(accg[mb][b][r], s, acc[mb][b][r]);
-            }
-            if constexpr (KQ == 1) {
-              __builtin_amdgcn_s_setprio(1);
-              __builtin_amdgcn_sched_barrier(0);
-            }
+          for (int b = 0; b < 2; b++)
+            accg[mb][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afcl[mb], bfc[b], accg[mb][b], 0, 0, 0);
+        if (j & 1) {
+          // The scaling reads the group's last MFMAs, so this wave has no
+          // MFMA to issue beside it: at the lower priority the other wave
+          // on the SIMD issues first (the C4 step 40.1-40.5 -> 39.1 ms;
+          // gate/up 407 -> 390-399 us, QKV 116 -> 106-111 us). With two k
+          // groups per workgroup the isolated block spilled more (18
+          // VGPRs, not 8-11), so they keep the interleave below. The
+          // lane's column scale of this group: bq[u] holds step u's two
+          // per lane column.
+          if constexpr (KQ == 1) {
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(0);
           }
-        } else {
 #pragma unroll
-          for (int mb = 0; mb < MB; mb++)
+          for (int b = 0; b < 2; b++) {
+            union { uint32_t u; half2_t h; } sc;
+            sc.u = bq[u][b].s;
+            const float s = (float)sc.h[j >> 1];
 #pragma unroll
-            for (int b = 0; b < 2; b++)
-              acc[mb][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[mb], bfc[b], acc[mb][b], 0, 0, 0);
+            for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+              for (int r = 0; r < 16; r++) acc[mb][b][r] = __builtin_fmaf(accg[mb][b][r], s, acc[mb][b][r]);
+          }
+          if constexpr (KQ == 1) {
+            __builtin_amdgcn_s_setprio(1);
+            __builtin_amdgcn_sched_barrier(0);
+          }
         }
-        if constexpr (EX && !FX) {
-          // the two correction products, each pass over every block, so no
-          // MFMA waits on the one just issued into the same accumulator
+      } else {
 #pragma unroll
-          for (int mb = 0; mb < MB; mb++)
+        for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-            for (int b = 0; b < 2; b++)
-              acc[mb][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afcl[mb], bfc[b], acc[mb][b], 0, 0, 0);
+          for (int b = 0; b < 2; b++)
+            acc[mb][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[mb], bfc[b], acc[mb][b], 0, 0, 0);
+      }
+      if constexpr (EX && !FX) {
+        // the two correction products, each pass over every block, so no
+        // MFMA waits on the one just issued into the same accumulator
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+          for (int b = 0; b < 2; b++)
+            acc[mb][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afcl[mb], bfc[b], acc[mb][b], 0, 0, 0);
+        if constexpr (FORM != TGOHIP_FORM_F16)
 #pragma unroll
           for (int mb = 0; mb < MB; mb++)
 #pragma unroll
             for (int b = 0; b < 2; b++)
               acc[mb][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afc[mb], bfcl[b], acc[mb][b], 0, 0, 0);
-        }
-        if constexpr (FX) {
-          // 8 MFMAs (64-row tiles), 4 LDS reads, the codes' 18 VALU; with
-          // two k groups an odd substep's 64 scaling fmas fill its VALU
-          // slots (with one, its MFMA region is scheduled freely, above)
-          if ((j & 1) == 0)
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-              __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
-              __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
-              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-              __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
-            }
-          else if (KQ == 2)
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
-              __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
-              __builtin_amdgcn_sched_group_barrier(0x002, 10, 0);  // VALU
-              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
-              __builtin_amdgcn_sched_group_barrier(0x002, 10, 0);  // VALU
-            }
-        } else if constexpr (EX) {
-          // 12 MFMAs (64-row tiles), 4 LDS reads, the B pairs' 36 VALU
+      }
+      if constexpr (FX) {
+        // 8 MFMAs (64-row tiles), 4 LDS reads, the codes' 18 VALU; with
+        // two k groups an odd substep's 64 scaling fmas fill its VALU
+        // slots (with one, its MFMA region is scheduled freely, above)
+        if ((j & 1) == 0)
 #pragma unroll
           for (int q = 0; q < 4; q++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
-            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // VALU
+            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // VALU
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
           }
-        } else {
+        else if (KQ == 2)
 #pragma unroll
           for (int q = 0; q < 4; q++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
-            __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // VALU
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // VALU
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // LDS read
+            __builtin_amdgcn_sched_group_barrier(0x002, 10, 0);  // VALU
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
+            __builtin_amdgcn_sched_group_barrier(0x002, 10, 0);  // VALU
           }
-        }
+      } else if constexpr (FORM == TGOHIP_FORM_F16) {
+        // no dequantization: 8 MFMAs (EX) or 4 and the next LDS reads
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++) {
-          afc[mb] = afn[mb];
-          afcl[mb] = afnl[mb];
+        for (int q = 0; q < 4; q++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+          if (EX) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
         }
+      } else if constexpr (EX) {
+        // 12 MFMAs (64-row tiles), 4 LDS reads, the B pairs' 36 VALU
 #pragma unroll
-        for (int b = 0; b < 2; b++) {
-          bfc[b] = bfn[b];
-          bfcl[b] = bfnl[b];
+        for (int q = 0; q < 4; q++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+          __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // VALU
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+          __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // VALU
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
         }
-        if (j == 1) {
-          __builtin_amdgcn_sched_barrier(0);
-          // vmcnt(2 * B loads + A DMA + scale DMA), expcnt untouched, lgkmcnt(0);
-          // vmcnt's low 4 bits sit at 3:0 and its high 2 at 15:14
-          constexpr int VMC = 2 * pipe_b_loads<FORM>() + AP * ACH + (LS ? 1 : 0);
-          static_assert(VMC < 64, "vmcnt fits 6 bits");
-          __builtin_amdgcn_s_waitcnt((VMC & 15) | ((VMC >> 4) << 14) | (7 << 4));
-          asm volatile("" ::: "memory");
-          __builtin_amdgcn_s_barrier();
-          asm volatile("" ::: "memory");
-          PIPE_DMA_A(kpos(kk + u + 3), (u + 3) % 4);
-          __builtin_amdgcn_sched_barrier(0);
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+          __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // VALU
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+          __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // VALU
         }
       }
-      __builtin_amdgcn_sched_barrier(0);
-      __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+      for (int mb = 0; mb < MB; mb++) {
+        afc[mb] = afn[mb];
+        afcl[mb] = afnl[mb];
+      }
+#pragma unroll
+      for (int b = 0; b < 2; b++) {
+        bfc[b] = bfn[b];
+        bfcl[b] = bfnl[b];
+      }
+      if (j == 1) {
+        __builtin_amdgcn_sched_barrier(0);
+        // vmcnt(2 * B loads + A DMA + scale DMA), expcnt untouched, lgkmcnt(0);
+        // vmcnt's low 4 bits sit at 3:0 and its high 2 at 15:14
+        constexpr int VMC = 2 * pipe_b_loads<FORM>() + AP * ACH + (LS ? 1 : 0);
+        static_assert(VMC < 64, "vmcnt fits 6 bits");
+        __builtin_amdgcn_s_waitcnt((VMC & 15) | ((VMC >> 4) << 14) | (7 << 4));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        PIPE_DMA_A(kpos(kk + u + 3), (u + 3) % 4);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(0);
+  };
+  typedef std::integral_constant<int, 0> U0;
+  typedef std::integral_constant<int, 1> U1;
+  typedef std::integral_constant<int, 2> U2;
+  typedef std::integral_constant<int, 3> U3;
+  if constexpr (TAIL) {
+    int kk = 0;
+    for (; kk + 4 <= nk; kk += 4) {
+      step(U0{}, kk);
+      step(U1{}, kk);
+      step(U2{}, kk);
+      step(U3{}, kk);
+    }
+    // K's last one to three k-steps (the loads past the end repeat the last one)
+    if (kk < nk) {
+      step(U0{}, kk);
+      if (kk + 1 < nk) step(U1{}, kk);
+      if (kk + 2 < nk) step(U2{}, kk);
+    }
+  } else {
+    for (int kk = 0; kk < nk; kk += 4) {
+      step(U0{}, kk);
+      step(U1{}, kk);
+      step(U2{}, kk);
+      step(U3{}, kk);
     }
   }
   __builtin_amdgcn_s_waitcnt(0);  // no DMA into LDS outlives the loop
@@ -1183,7 +941,7 @@ __global__ void repack_kernel(RepackArgs a) {
   for (int j = 0; j < 4; j++) {
     const int kb = ks * 64 + 16 * j + 8 * h;
     if (FORM == TGOHIP_FORM_F16) {
-      uint16_t* dst = (uint16_t*)a.wp + ot * 32 + j * 8;
+      uint16_t* dst = (uint16_t*)a.wp + ((ot / 64 * 4 + j) * 64 + lane) * 8;
       for (int e = 0; e < 8; e++) dst[e] = ((const uint16_t*)a.plane)[(size_t)(kb + e) * N + n];
     } else if (FORM == TGOHIP_FORM_I4_SYM) {
       uint32_t w = 0;
@@ -1208,8 +966,9 @@ __global__ void repack_kernel(RepackArgs a) {
         const uint32_t b = (uint32_t)((int)((const int8_t*)a.plane)[i] + 128) & 255u;
         w[e >> 2] |= b << (8 * byte_slot(e & 3));
       }
-      ((uint32_t*)a.wp)[ot * 8 + j * 2] = w[0];
-      ((uint32_t*)a.wp)[ot * 8 + j * 2 + 1] = w[1];
+      uint32_t* dst = (uint32_t*)a.wp + ((ot / 64 * 2 + j / 2) * 64 + lane) * 4 + (j & 1) * 2;
+      dst[0] = w[0];
+      dst[1] = w[1];
     }
     // per-k scales (and zeros) for I8 / I4_TGO: written by lanes 0 and 32.
     if ((FORM == TGOHIP_FORM_I8 || FORM == TGOHIP_FORM_I4_TGO) && (lane & 31) == 0) {
@@ -1748,9 +1507,10 @@ static int choose_pipe_splits(int tiles, int KS, int slots) {
 // (at 128 rows: 45.6 us unsplit against 45.4 us plus a 7 us reduction).
 // The exact (EX) kernel runs 64-row tiles 4 waves wide at every M: its A ring
 // holds two planes, and at 128 rows its fragments would not fit the registers.
+// So do f16 weights, whose fragments in flight take 96 registers.
 static void pipe_shape(const PackedWeight& w, int M, int ncu, int& mw, int& nw, int& tiles_n,
                        int& tiles, int& splits, int epi = EPI_F32, bool ex = false) {
-  mw = (M <= 384 || ex) ? 64 : 128;
+  mw = (M <= 384 || ex || w.form == TGOHIP_FORM_F16) ? 64 : 128;
   const int nb = w.N / 32, rows = (M + mw - 1) / mw;
   nw = 4;
   if (mw == 128) {
@@ -1778,6 +1538,12 @@ static void pipe_shape(const PackedWeight& w, int M, int ncu, int& mw, int& nw, 
     else if (tiles > slots && 5 * tiles < 8 * slots) splits = 2;
     while (splits > 1 && (w.K / 64) / splits < 8) splits--;
   }
+  // Exact tiles that leave CUs without a workgroup even so go on to one per
+  // CU, in shorter runs of K (at least 6 k-steps): [12288, 4096] of symmetric
+  // int4 at 48 rows 8 -> 16 splits 28.5 -> 22.1 us, [1600, 4096] at 96 rows 3 -> 4
+  // splits 17.6 -> 14.5 (without the reduction). With f16 operands, whose
+  // k-steps are shorter, 16 splits cost [12288, 4096] 21.0 -> 22.4 with it.
+  while (ex && splits > 1 && splits < 16 && tiles * (splits + 1) <= ncu && (w.K / 64) / (splits + 1) >= 6) splits++;
   if (ex && pipe_ex_splits() > 0) {
     splits = pipe_ex_splits();
     while (splits > 1 && (w.K / 64) / splits < 8) splits--;
@@ -1797,8 +1563,20 @@ template <int FORM, int MW, int NW, int KQ = 1, bool EX = false>
 static void launch_pipe_form(const GemmArgs& g, int epi, dim3 grid, int tiles_n, int tiles,
                              int cm, int xs, const QKRopeArgs& qa, hipStream_t st) {
   const dim3 blk(64 * NW * KQ);
-#define PIPE_LAUNCH(E) \
-  hipLaunchKernelGGL((gemm_pipe_kernel<FORM, E, MW, NW, KQ, EX>), grid, blk, 0, st, g, tiles_n, tiles, cm, xs, qa)
+  constexpr bool FX = EX && FORM == TGOHIP_FORM_I4_SYM;
+  const bool whole = FX && (g.K / 64) % 4 == 0;
+#define PIPE_LAUNCH(E)                                                                            \
+  do {                                                                                            \
+    if constexpr (FX)                                                                             \
+      if (whole) {                                                                                \
+        hipLaunchKernelGGL((gemm_pipe_kernel<FORM, E, MW, NW, KQ, EX, false>), grid, blk, 0, st, g, \
+                           tiles_n, tiles, cm, xs, qa);                                           \
+        break;                                                                                    \
+      }                                                                                           \
+    if constexpr (!FX || KQ == 1) /* two k groups go with whole groups of four */                 \
+      hipLaunchKernelGGL((gemm_pipe_kernel<FORM, E, MW, NW, KQ, EX>), grid, blk, 0, st, g, tiles_n, \
+                         tiles, cm, xs, qa);                                                      \
+  } while (0)
   switch (epi) {
     case EPI_F32: PIPE_LAUNCH(EPI_F32); break;
     case EPI_F16: PIPE_LAUNCH(EPI_F16); break;
@@ -1818,7 +1596,8 @@ static void launch_pipe_shape(const GemmArgs& g, int epi, dim3 grid, int mw, int
   if (ex && kq == 2) launch_pipe_form<FORM, 64, 4, 2, true>(g, epi, grid, tiles_n, tiles, cm, xs, qa, st);
   else if (ex) launch_pipe_form<FORM, 64, 4, 1, true>(g, epi, grid, tiles_n, tiles, cm, xs, qa, st);
   else if (mw == 64 && kq == 2) launch_pipe_form<FORM, 64, 4, 2>(g, epi, grid, tiles_n, tiles, cm, xs, qa, st);
-  else if (mw == 64) launch_pipe_form<FORM, 64, 4>(g, epi, grid, tiles_n, tiles, cm, xs, qa, st);
+  else if (FORM == TGOHIP_FORM_F16 || mw == 64) launch_pipe_form<FORM, 64, 4>(g, epi, grid, tiles_n, tiles, cm, xs, qa, st);
+  else if constexpr (FORM == TGOHIP_FORM_F16) return;
   else if (nw == 8) launch_pipe_form<FORM, 128, 8>(g, epi, grid, tiles_n, tiles, cm, xs, qa, st);
   else launch_pipe_form<FORM, 128, 4>(g, epi, grid, tiles_n, tiles, cm, xs, qa, st);
 }
@@ -1847,19 +1626,23 @@ static PipeLaunch pipe_launch(const PackedWeight& w, int M, int ncu, int epi, bo
   // group (O and down at 128 rows, 8 splits of 8 and 24 k-steps, ran 6% and
   // 2% slower with two).
   p.kq = (p.mw == 64 && p.splits == 1 && p.tiles <= ncu && KS % 8 == 0 && pipe_kq_enabled()) ? 2 : 1;
-  // whole groups of 4 k-steps per split and k group (KS is a multiple of 4)
+  // whole groups of 4 k-steps per split and k group; the last split takes
+  // what is left of K
   p.ksteps_per_split = ((KS + p.splits - 1) / p.splits + 4 * p.kq - 1) / (4 * p.kq) * (4 * p.kq);
   p.splits = (KS + p.ksteps_per_split - 1) / p.ksteps_per_split;
   return p;
 }
 
 // xlo: the lo plane of an XK_X2 activation (the exact kernel), or null.
+// whole > 0: these M rows are a band of a call over `whole` rows and take that
+// call's tile shape and splits, so that their sums are the whole call's.
 static int gemm_pipe_enqueue(const PackedWeight& w, const void* x, const void* xlo, int M, void* y,
                              int epi, float* workspace, size_t ws_bytes, int ncu, hipStream_t st,
-                             int* defer, const QKRopeArgs* qa = nullptr) {
+                             int* defer, const QKRopeArgs* qa = nullptr, int whole = 0) {
   const bool ex = xlo != nullptr;
-  const PipeLaunch pl = pipe_launch(w, M, ncu, epi, ex);
-  const int mw = pl.mw, nw = pl.nw, tiles_n = pl.tiles_n, tiles = pl.tiles, kq = pl.kq;
+  const PipeLaunch pl = pipe_launch(w, whole > 0 ? whole : M, ncu, epi, ex);
+  const int mw = pl.mw, nw = pl.nw, tiles_n = pl.tiles_n, kq = pl.kq;
+  const int tiles = tiles_n * ((M + mw - 1) / mw);
   int splits = pl.splits;
   GemmArgs g{};
   g.x = x;
@@ -1888,6 +1671,9 @@ static int gemm_pipe_enqueue(const PackedWeight& w, const void* x, const void* x
   // (262 -> 250 us for the C4 LM head at 136 rows).
   const int cm = tiles / tiles_n <= 4 ? 1 : 0;
   switch (w.form) {
+    case TGOHIP_FORM_F16:
+      launch_pipe_shape<TGOHIP_FORM_F16>(g, epi, grid, mw, nw, kq, tiles_n, tiles, cm, xs, ex, qa ? *qa : QKRopeArgs{}, st);
+      break;
     case TGOHIP_FORM_I4_SYM:
       launch_pipe_shape<TGOHIP_FORM_I4_SYM>(g, epi, grid, mw, nw, kq, tiles_n, tiles, cm, xs, ex, qa ? *qa : QKRopeArgs{}, st);
       break;
@@ -1915,32 +1701,113 @@ static int pipe_min_rows() {
   return v;
 }
 
-// The pipelined kernel serves the int4 packs and int8 with f16 activations
-// or activation pairs (XK_X2, the exact kernel); f16 weights and unsplit f32
-// activations use gemm_kernel.
+// The pipelined kernel serves f16 activations and activation pairs (XK_X2, the
+// exact kernel); an f32 activation is split into a pair first
+// (gemm_enqueue_f32).
 static bool use_pipe(const PackedWeight& w, int xk, int M) {
-  return xk != XK_F32 && w.form != TGOHIP_FORM_F16 && M >= pipe_min_rows() &&
-         (w.K / 64) % 4 == 0 &&
+  // f16 operands over f16 weights keep gemm_kernel's 128-row tiles where these
+  // fill the chip or K is long: [4096, 24576] at 1100 rows 260 us against 297,
+  // [12288, 4096] at 500 rows 74 against 78; else [5120, 10240] at 1100 rows
+  // 172 -> 160, [4096, 6144] 97 -> 77.
+  if (xk == XK_F16 && w.form == TGOHIP_FORM_F16 && M > 384 &&
+      (w.K >= 8192 || (int64_t)((w.N + 255) / 256) * ((M + 127) / 128) >= 512))
+    return false;
+  // f32 rows over a small grid of f16 or symmetric int4 weights: the pair's own
+  // launch costs more than gemm_kernel's 32-row tiles ([4096, 6144] at 48 rows
+  // 22.1 us against 23.9, at 96 28.3 against 30.7; N = 24576 46.8 -> 41.4, 78 -> 64;
+  // the other packs gain at N = 6144 too, 29.4 -> 26.4).
+  if (xk == XK_F32 && M <= 96 && w.N <= 8192 && (w.form == TGOHIP_FORM_F16 || w.form == TGOHIP_FORM_I4_SYM))
+    return false;
+  // up to 64 rows over a small grid of f16 weights likewise ([12288, 4096] at 48
+  // f16 rows 29.9 us against 34.2, [4096, 6144] 22.4 against 24.3)
+  if (w.form == TGOHIP_FORM_F16 && M <= 64 && w.N <= 8192) return false;
+  return M >= pipe_min_rows() &&
          (int64_t)M * w.K < ((int64_t)1 << 31);  // its activation offsets are 32-bit
 }
 
-// Workspace bytes a call needs for split-K partials: xk < 0 bounds every
-// activation type and epilogue; otherwise the bytes of exactly the call
-// gemm_enqueue makes over that activation type with an f32 or f16 epilogue.
-size_t gemm_workspace_bytes(const PackedWeight& w, int M, int ncu, int xk) {
-  if (M <= 0) return 0;  // nothing launches (and no tiles to divide the slots by)
-  const int MW = small_mw(w, M, ncu);
-  int s;
-  if (xk < 0) {
-    s = std::max({choose_splits(M, w.N, w.K, MW, ncu), pipe_launch(w, M, ncu, EPI_F32, false).splits,
-                  pipe_launch(w, M, ncu, EPI_F32, true).splits});
-  } else if (use_pipe(w, xk, M)) {
-    s = pipe_launch(w, M, ncu, EPI_F32, xk == XK_X2).splits;
-  } else if (use_gemv(w, xk, M, ncu)) {
-    s = 1;
-  } else {
-    s = choose_splits(M, w.N, w.K, MW, ncu);  // gemm_kernel's grid.z
+// gemm_rows_kernel's launch for a call: cb column blocks per workgroup (0: it
+// does not serve the call) and K in `splits`. Both sides of each line were
+// measured over every form (us, start of the line's other kernel -> rows):
+//  * up to 16 f32 or pair rows, staged in LDS beside the waves' sums: all
+//    shapes with up to 8 rows ([4096, 6144] of symmetric int4 12.1 -> 7.6 at one
+//    row, [4096, 24576] 24.2 -> 19.3, [4096, 151936] 120 -> 90; int8 [5120,
+//    10240] at one row 21.6 -> 19.6); with 9 to 16 rows [4096, 24576] of f16
+//    weights 45.8 -> 37.7, of symmetric int4 27.0 -> 26.4. Shares of K that
+//    don't fit go to splits of it ([25600, 5120] at 4 rows: 4, 31.8 -> 27.7),
+//    and a K of 8192 or more over few column blocks takes two ([12288, 4096]
+//    at one row 16.2 -> 12.8, unsplit 14.2).
+//  * f16 operands up to 32 rows stay with gemm_gemv_kernel where it stages the
+//    rows, and elsewhere but for long K (symmetric int4 from 5120, the other
+//    packs 8192 to 16384 at 4 rows and more: [12288, 4096] at 8 rows 25.9 -> 18.2)
+//    and for a K that leaves that kernel fewer than four waves ([5504, 3584] of
+//    int8 at 2 rows, one wave: 57 us).
+//  * otherwise while all workgroups together read at most 64 MB of activations
+//    (80 above 32 rows): [1024, 6144] pairs at 32 rows (25 MB) 11.6 -> 6.7 and at 67
+//    (53 MB) 17.3 -> 13.6; at 128 (100 MB) 19.1 -> 19.0, and [4096, 6144] at 40
+//    (126 MB) 19.5 -> 28. A launch of under half the CUs splits K from 2048 up
+//    ([4096, 1024] at 67 rows 31.8 -> 13.1; [1024, 1024] 9.6 -> 10.2).
+struct RowsShape {
+  int cb, splits;
+};
+static RowsShape rows_shape(const PackedWeight& w, int xk, int M, int epi, int ncu) {
+  const bool sw = epi == EPI_SWIGLU_F16 || epi == EPI_SWIGLU_X2;
+  RowsShape r{0, 1};
+  const int KS = w.K / 64, cb = sw ? 2 : 1;
+  const int groups = (w.N / 32 + cb - 1) / cb * (M > 32 ? (M + 63) / 64 : 1);
+  // the planes of a split fit the allocation-free linear's array
+  auto planes_fit = [&](int s) {
+    return s == 1 || (size_t)s * split_plane_stride(M, w.N) * sizeof(float) <= kRowsPlaneBytes;
+  };
+  if (xk != XK_F16 && M <= 16) {
+    int s = groups * 2 <= ncu && KS >= 128 ? 2 : 1;
+    while (!rows_staged(M, (KS + s - 1) / s) && s < 16) s *= 2;
+    const bool packed8 = w.form == TGOHIP_FORM_I8 || w.form == TGOHIP_FORM_I4_TGO;
+    if (rows_staged(M, (KS + s - 1) / s) && planes_fit(s) && !(packed8 && s >= 8 && M > 8)) {
+      r.cb = cb;
+      r.splits = s;
+      return r;
+    }
   }
+  if (xk == XK_F16 && M <= 32 && w.form != TGOHIP_FORM_F16) {
+    const GemvShape gv = gemv_shape(w, EPI_F32, M, ncu);
+    if (gv.staged) return r;
+    if (gv.w >= 4 && (w.form == TGOHIP_FORM_I4_SYM ? KS < 80 : (M < 4 || KS < 128 || KS > 256))) return r;
+  }
+  if (sw && M > 32 && w.form != TGOHIP_FORM_F16) return r;
+  const int64_t traffic = (int64_t)(w.N / 32 + cb - 1) / cb * M * w.K * (xk == XK_F16 ? 2 : 4);
+  // half of that where a second round of workgroups would be mostly empty
+  // ([5120, 10240] at 16 f16 rows, 320 column blocks, 52 MB: 27.0 us against 29.1)
+  const int64_t most = (int64_t)(groups > ncu && groups < 2 * ncu && M <= 32 ? 40 : M <= 32 ? 64 : 80) * 1000000;
+  if (traffic > most) return r;
+  r.cb = cb;
+  if (KS >= 32)
+    while (r.splits < 8 && groups * r.splits * 2 <= ncu && KS / (r.splits * 2) >= 8 && planes_fit(r.splits * 2))
+      r.splits *= 2;
+  return r;
+}
+
+// Bytes of split-K planes that linear_noalloc's limit applies to: the splits
+// of gemm_kernel's and the pipelined kernel's tiles, none on the small-M
+// kernel. What the call itself writes is no more than this or the limit.
+size_t gemm_limit_bytes(const PackedWeight& w, int M, int ncu, int xk) {
+  if (M <= 0) return 0;  // nothing launches (and no tiles to divide the slots by)
+  int s;
+  if (xk != XK_F32 && w.form != TGOHIP_FORM_F16 && (w.K / 64) % 4 == 0 && use_pipe(w, xk, M))
+    s = pipe_launch(w, M, ncu, EPI_F32, xk == XK_X2).splits;
+  else if (use_gemv(w, xk, M, ncu))
+    s = 1;
+  else
+    s = choose_splits(M, w.N, w.K, small_mw(w, M, ncu), ncu);
+  return s > 1 ? (size_t)s * split_plane_stride(M, w.N) * sizeof(float) : 0;
+}
+
+// The most workspace a call over M rows uses for split-K planes, whatever its
+// activation and epilogue.
+size_t gemm_workspace_bytes(const PackedWeight& w, int M, int ncu) {
+  if (M <= 0) return 0;
+  int s = std::max({choose_splits(M, w.N, w.K, small_mw(w, M, ncu), ncu),
+                    pipe_launch(w, M, ncu, EPI_F32, false).splits, pipe_launch(w, M, ncu, EPI_F32, true).splits});
+  for (int xk : {XK_F16, XK_F32, XK_X2}) s = std::max(s, rows_shape(w, xk, M, EPI_F32, ncu).splits);
   return s > 1 ? (size_t)s * split_plane_stride(M, w.N) * sizeof(float) : 0;
 }
 
@@ -1962,6 +1829,72 @@ int gemm_enqueue_qkrope(const PackedWeight& w, const void* x, int M, const QKRop
   return gemm_pipe_enqueue(w, x, xlo, M, nullptr, EPI_QKROPE, nullptr, 0, ncu, st, nullptr, &qa);
 }
 
+// x [n] f32 -> the activation pair at out: n halves f16(x), then n halves
+// f16(x - f16(x)). Eight elements per thread; n is a multiple of 64.
+__global__ __launch_bounds__(256) void split_pair_kernel(const float* x, half_t* out, size_t n) {
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
+  if (i >= n) return;
+  const float4_t a = *(const float4_t*)(x + i), b = *(const float4_t*)(x + i + 4);
+  const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  half8_t hi, lo;
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    hi[e] = (half_t)v[e];
+    lo[e] = (half_t)(v[e] - (float)hi[e]);
+  }
+  *(half8_t*)(out + i) = hi;
+  *(half8_t*)(out + n + i) = lo;
+}
+
+// f32 activations on the pipelined kernel: split into a pair in the workspace
+// once, then the exact kernel, instead of gemm_kernel, which splits them again
+// in every workgroup, takes three MFMAs per product for symmetric int4 too and
+// spills 76-211 VGPRs with 128-row tiles of the other packs ([4096, 12288] of
+// tgo's int4 over 353 f32 rows: 541 us before). The pair and the split-K planes
+// share the workspace; where they don't fit, the rows go in bands, each with
+// the whole call's tile shape and splits, so the bands don't change the sums.
+static size_t f32_band_bytes(const PackedWeight& w, const PipeLaunch& pl, int rows) {
+  const size_t planes = pl.splits > 1 ? (size_t)pl.splits * split_plane_stride(rows, w.N) * sizeof(float) : 0;
+  return planes + (size_t)rows * w.K * sizeof(float);
+}
+// The most rows, up to M, whose band fits `bytes`: whole row tiles, or fewer
+// rows than one tile; 0 when not even one row fits.
+static int f32_band_rows(const PackedWeight& w, const PipeLaunch& pl, int M, size_t bytes) {
+  if (f32_band_bytes(w, pl, M) <= bytes) return M;
+  int lo = 0, hi = M;  // band_bytes grows with the rows
+  while (hi - lo > 1) {
+    const int mid = lo + (hi - lo) / 2;
+    if (f32_band_bytes(w, pl, mid) <= bytes) lo = mid;
+    else hi = mid;
+  }
+  return lo >= pl.mw ? lo / pl.mw * pl.mw : lo;
+}
+constexpr size_t kPairBytes = (size_t)64 << 20;  // most bytes of pair tgohip_linear's workspace holds
+size_t gemm_f32_workspace_bytes(const PackedWeight& w, int M, int ncu) {
+  if (M <= 0 || !use_pipe(w, XK_F32, M)) return 0;
+  const PipeLaunch pl = pipe_launch(w, M, ncu, EPI_F32, true);
+  const int64_t most = std::max<int64_t>(pl.mw, (int64_t)(kPairBytes / sizeof(float)) / w.K / pl.mw * pl.mw);
+  return f32_band_bytes(w, pl, (int)std::min<int64_t>(M, most));
+}
+static int gemm_enqueue_f32(const PackedWeight& w, const float* x, int M, void* y, int epi,
+                            float* workspace, size_t ws_bytes, int ncu, hipStream_t st) {
+  const PipeLaunch pl = pipe_launch(w, M, ncu, epi, true);
+  const int band = workspace ? f32_band_rows(w, pl, M, ws_bytes) : 0;
+  if (band <= 0) return fail(TGOHIP_ESTATE, "linear: the workspace holds no band of the split activation");
+  const size_t out = epi == EPI_F16 ? sizeof(half_t) : sizeof(float);
+  for (int r0 = 0; r0 < M; r0 += band) {
+    const int rows = std::min(band, M - r0);
+    const size_t n = (size_t)rows * w.K, planes = f32_band_bytes(w, pl, rows) - n * sizeof(float);
+    half_t* pair = (half_t*)((char*)workspace + planes);
+    hipLaunchKernelGGL(split_pair_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, st,
+                       x + (size_t)r0 * w.K, pair, n);
+    const int rc = gemm_pipe_enqueue(w, pair, pair + n, rows, (char*)y + (size_t)r0 * w.N * out, epi,
+                                     workspace, planes, ncu, st, nullptr, nullptr, M);
+    if (rc) return rc;
+  }
+  return 0;
+}
+
 int gemm_enqueue(const PackedWeight& w, const void* x, int xk, int M, void* y, int epi,
                  float* workspace, size_t ws_bytes, int ncu, hipStream_t st, int* defer) {
   if (defer) *defer = 0;
@@ -1973,7 +1906,38 @@ int gemm_enqueue(const PackedWeight& w, const void* x, int xk, int M, void* y, i
     return fail(TGOHIP_ESTATE, "linear: the activation-pair SwiGLU output goes with activation-pair input");
   // an activation pair's lo plane follows its hi plane
   const void* xlo = xk == XK_X2 ? (const void*)((const half_t*)x + (size_t)M * w.K) : nullptr;
-  if (use_pipe(w, xk, M))
+  // A QKV projection (the deferring f32 call) whose derived-rows form fuses its
+  // epilogue keeps the same kernel here, so that both give the same bits.
+  const bool fusable = defer && epi == EPI_F32 && xk == XK_X2 && gemm_qkrope_fusable(w, M, ncu);
+  const RowsShape rs = rows_shape(w, xk, M, epi, ncu);
+  if (rs.cb && !fusable) {
+    GemmArgs g{};
+    g.x = x;
+    g.xlo = xlo;
+    g.wp = w.wp;
+    g.ws = w.ws;
+    g.wz = w.wz;
+    g.y = y;
+    g.M = M;
+    g.K = w.K;
+    g.N = w.N;
+    g.ksteps_per_split = (w.K / 64 + rs.splits - 1) / rs.splits;
+    const int splits = (w.K / 64 + g.ksteps_per_split - 1) / g.ksteps_per_split;
+    if (splits > 1) {
+      if (!workspace || ws_bytes < (size_t)splits * split_plane_stride(M, w.N) * sizeof(float))
+        return fail(TGOHIP_ESTATE, "linear: split-K workspace too small");
+      g.part = workspace;
+      g.pstride = split_plane_stride(M, w.N);
+    }
+    launch_gemm_rows(w.form, g, xk, epi, rs.cb, splits, st);
+    if (defer) *defer = splits > 1 ? splits : 0;
+    if (splits > 1 && !defer) launch_reduce(g, epi, splits, st);
+    TGOHIP_HIP(hipGetLastError());
+    return 0;
+  }
+  if (xk == XK_F32 && (epi == EPI_F32 || epi == EPI_F16) && !defer && use_pipe(w, xk, M))
+    return gemm_enqueue_f32(w, (const float*)x, M, y, epi, workspace, ws_bytes, ncu, st);
+  if (xk != XK_F32 && use_pipe(w, xk, M))
     return gemm_pipe_enqueue(w, x, xlo, M, y, epi, workspace, ws_bytes, ncu, st, defer);
   if (use_gemv(w, xk, M, ncu)) {
     GemmArgs g{};

@@ -468,7 +468,7 @@ int place_weight(tgohip_ctx* c, PortKind kind, int l, int form, int K, int N, co
   return 0;
 }
 
-int ensure_activations(tgohip_ctx* c, int rows, int B) {
+int ensure_activations(tgohip_ctx* c, int rows, int B, int head_rows) {
   const tgohip_model_cfg& m = c->cfg;
   const size_t d = m.hidden, qw = (size_t)m.heads * m.head_dim, kw = (size_t)m.kv_heads * m.head_dim;
   const size_t f = m.ffn;
@@ -498,7 +498,7 @@ int ensure_activations(tgohip_ctx* c, int rows, int B) {
   for (const Layer& L : c->layers)
     for (const PackedWeight* w : {&L.qkv, &L.wo, &L.gateup, &L.down})
       if (w->form >= 0) ws = std::max(ws, gemm_workspace_bytes(*w, rows, c->ncu));
-  if (c->lm_head.form >= 0) ws = std::max(ws, gemm_workspace_bytes(c->lm_head, B, c->ncu));
+  if (c->lm_head.form >= 0) ws = std::max(ws, gemm_workspace_bytes(c->lm_head, head_rows, c->ncu));
   if ((rc = c->gemm_ws.ensure(ws + 256))) return rc;
   return 0;
 }
@@ -998,7 +998,7 @@ int step_launch(tgohip_ctx* c, const tgohip_batch_step* s, StepLaunch& o) {
   const bool compact = nh > 0 && nh < B;
   if (!compact) c->head_rows.clear();
   const int HB = compact ? nh : B;  // rows of the head
-  if ((rc = ensure_activations(c, Tw, B))) return rc;
+  if ((rc = ensure_activations(c, Tw, B, HB))) return rc;
   if ((rc = ensure_attn_parts(c, plan.parts))) return rc;
 
   // One staged upload of every port (batch.go:385-405).
@@ -1400,7 +1400,8 @@ int tgohip_linear(tgohip_ctx* c, int handle, const void* x, int x_dtype, int M, 
   if (!w) return TGOHIP_EINVAL;
   if (M < 0) return fail(TGOHIP_EINVAL, "linear: M is " + std::to_string(M));
   if (M == 0) return 0;  // an empty batch: nothing to launch
-  const size_t ws = gemm_workspace_bytes(*w, M, c->ncu);
+  size_t ws = gemm_workspace_bytes(*w, M, c->ncu);
+  if (xkind(x_dtype) == XK_F32) ws = std::max(ws, gemm_f32_workspace_bytes(*w, M, c->ncu));
   int rc = c->gemm_ws.ensure(ws + 256);
   if (rc) return rc;
   return gemm_enqueue(*w, x, xkind(x_dtype), M, y,
@@ -1417,8 +1418,7 @@ int tgohip_linear_noalloc(tgohip_ctx* c, int handle, const void* x, int x_dtype,
   if (!w) return TGOHIP_EINVAL;
   if (M < 0) return fail(TGOHIP_EINVAL, "linear_noalloc: M is " + std::to_string(M));
   if (M == 0) return 0;  // an empty batch: nothing to launch
-  // exactly what this call's kernels use (its activation type decides them)
-  const size_t ws = gemm_workspace_bytes(*w, M, c->ncu, xkind(x_dtype));
+  const size_t ws = gemm_limit_bytes(*w, M, c->ncu, xkind(x_dtype));
   if (ws > kScratchBytes)
     return fail(TGOHIP_EINVAL, "linear_noalloc: M = " + std::to_string(M) + " over [" +
                                    std::to_string(w->K) + "," + std::to_string(w->N) +
@@ -1435,7 +1435,7 @@ int tgohip_linear_workspace(tgohip_ctx* c, int handle, int x_dtype, int M, size_
   PackedWeight* w = handle_of(c, handle);
   if (!w) return TGOHIP_EINVAL;
   if (M < 0) return fail(TGOHIP_EINVAL, "linear_workspace: M is " + std::to_string(M));
-  *bytes = gemm_workspace_bytes(*w, M, c->ncu, xkind(x_dtype));
+  *bytes = gemm_limit_bytes(*w, M, c->ncu, xkind(x_dtype));
   return 0;
 }
 
@@ -1866,7 +1866,7 @@ int tgohip_sched_submit(tgohip_sched* s, int32_t* out_slot, int32_t* out_done,
   }
   tgohip_batch_step bs{total, n, maxp, s->ids.data(), nullptr, nullptr, nullptr,
                        s->lengths.data(), s->extents.data(), s->last.data(), s->table.data()};
-  if ((rc = ensure_activations(c, total, n))) return rc;  // argmax holds n entries from here
+  if ((rc = ensure_activations(c, total, n, n))) return rc;  // argmax holds n entries from here
   StepLaunch o;
   o.feed = (const int32_t*)c->argmax.p;
   o.keep_idle = 1;
