@@ -388,3 +388,44 @@ def test_c5_shaped_shared_prefix_every_row(ctx, torch_gpu):
     # running maxima: each is within 2^-11 of exact, so they agree to 2^-10
     rel = np.abs(shared - plain).max() / np.abs(plain).max()
     assert rel <= 2.0 ** -10, rel
+
+
+@pytest.mark.parametrize("lengths,extents", [
+    ([2048, 2049, 4096, 4097, 6145], [1, 1, 1, 1, 1]),   # decode items: whole, 2, 2, 3 and 4 parts
+    ([3072, 3073, 6170], [20, 40, 33]),                  # prefill items: whole, 2 and 3 parts
+    ([2049, 3100, 64, 1], [1, 40, 40, 1]),               # both kinds
+])
+@pytest.mark.parametrize("q_f16", [False, True])
+def test_contexts_split_into_even_parts(ctx, torch_gpu, lengths, extents, q_f16):
+    """Contexts at and just past the longest part: a sequence's positions go into equal
+    parts of whole tiles. Every row against the oracle, and every sequence equal to the
+    bit to the same sequence alone."""
+    H, Hkv, block = 8, 2, 16
+    rng = np.random.default_rng(sum(lengths))
+    need = [(n + block - 1) // block for n in lengths]
+    perm = rng.permutation(sum(need))
+    maxp = max(need)
+    pages = np.zeros((len(lengths), maxp), np.uint32)
+    at = 0
+    for s, n in enumerate(need):
+        pages[s, :n] = perm[at:at + n]
+        at += n
+    k16, v16 = (rng.standard_normal((at * block, Hkv, DH)).astype(np.float16).view(np.uint16)
+                for _ in range(2))
+    q = rng.standard_normal((sum(extents), H, DH)).astype(np.float32)
+    if q_f16:
+        q = q.astype(np.float16).astype(np.float32)
+    scale = 1.0 / math.sqrt(DH)
+    args = (k16, v16)
+    got = run(ctx, torch_gpu, q, *args, lengths, extents, pages.ravel(), maxp, block, scale, H, Hkv,
+              q_f16=q_f16)
+    want, b = oracle.ragged_attention_f64(q, H, Hkv, DH, k16, v16, lengths, extents,
+                                          pages.ravel().tolist(), maxp, block, scale)
+    err = np.abs(got - want).max()
+    assert err <= budget(b), (err, budget(b), b)
+    at = 0
+    for s, n in enumerate(extents):
+        alone = run(ctx, torch_gpu, q[at:at + n], *args, [lengths[s]], [n], pages[s], maxp, block,
+                    scale, H, Hkv, q_f16=q_f16)
+        assert np.array_equal(alone, got[at:at + n]), s
+        at += n

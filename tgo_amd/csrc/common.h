@@ -66,8 +66,8 @@ struct AttnCombine {
 };
 
 constexpr int kAttnTile = 64;     // positions staged in LDS per iteration
-constexpr int kAttnSplitDecode = 2560;   // positions per part of a split decode-style item
-constexpr int kAttnSplitPrefill = 2048;  // positions per part of a split prefill-style item
+constexpr int kAttnSplitDecode = 2048;   // most positions per part of a split decode-style item
+constexpr int kAttnSplitPrefill = 3072;  // most positions per part of a split prefill-style item
 constexpr int kAttnSplitShared = 512;    // positions per part of a shared-prefix item
 constexpr int kAttnRowsP = 128;   // rows per prefill-style item (4 waves x 32)
 constexpr int kHeadDim = 128;
@@ -297,6 +297,8 @@ void launch_quantize_i8(const float* w, size_t n, int8_t* q, uint16_t* scales, h
 void launch_quantize_i4tgo(const float* w, size_t n, uint32_t* codes, uint16_t* scales,
                            uint16_t* zeros, hipStream_t st);
 void launch_synth_gain(uint64_t seed, uint64_t stream, size_t n, float* out, hipStream_t st);
+// Copies whole 16-byte words from pinned host memory (device-visible) to dst.
+void launch_fetch(const void* host, void* dst, size_t bytes, hipStream_t st);
 void launch_fill_f32(float* p, size_t n, float v, hipStream_t st);
 
 // ---- peak probes (kernels/probe.hip) ---------------------------------------

@@ -519,6 +519,15 @@ __device__ __forceinline__ void attn_decode(const AttnArgs& a, const AttnItem& i
 //   16t + (e < 4 ? 4kh + e : 8 + 4kh + e - 4) of the block, which is exactly
 //   where the lane's own probabilities sit (scores i = 8t..8t+7), so P never
 //   leaves registers; the A operand is two 8-byte reads of transposed V.
+// LDS operands read ahead of their MFMAs, in fragments (K: one read each, V:
+// two). What bounds a prefill item is its MFMAs (32 a tile and wave with f16 q,
+// 64 with f32) and its softmax's VALU (32 quarter-rate exponentials of about
+// half its time), which overlap only in part; with the reads ahead neither
+// waits for LDS: 8 chunks of 256 beside 56 decode rows, f32 q, 204 -> 199 us,
+// four chunks of 512 with f16 q 128 -> 126.
+constexpr int kAttnKAhead = 4;
+constexpr int kAttnVAhead = 2;
+
 template <int BLK, bool QF16>
 __device__ __forceinline__ void attn_prefill(const AttnArgs& a, const AttnItem& it, const AttnCtx& c,
                                              char* smem) {
@@ -565,21 +574,27 @@ __device__ __forceinline__ void attn_prefill(const AttnArgs& a, const AttnItem& 
     attn_store_tile(c, Ks, Vs, kr, vr);
     attn_lds_barrier();
     if (t0 + kAttnTile < it.kv_hi) attn_load_tile<BLK>(a, c, t0 + kAttnTile, it.kv_hi, kr, vr);
-    float16_t sc[2];
+    // The two position blocks' chains side by side (an MFMA does not wait for
+    // the one just issued into the same sums), K fragments kAttnKAhead reads
+    // ahead of their MFMAs; left to itself the scheduler reads two and waits
+    // for them before each pair of MFMAs.
+    float16_t sc[2] = {};
 #pragma unroll
-    for (int pb = 0; pb < 2; pb++) {
-      float16_t acc;
+    for (int ss = 0; ss < 8; ss++)
 #pragma unroll
-      for (int i = 0; i < 16; i++) acc[i] = 0.f;
-      const int pos = pb * 32 + l32;
-#pragma unroll
-      for (int ss = 0; ss < 8; ss++) {
+      for (int pb = 0; pb < 2; pb++) {
+        const int pos = pb * 32 + l32;
         const half8_t ka = *(const half8_t*)(Ks + (pos * 16 + ((2 * ss + kh) ^ (pos & 15))) * 8);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qh[ss], acc, 0, 0, 0);
-        if (!QF16) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, ql[ss], acc, 0, 0, 0);
+        sc[pb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, qh[ss], sc[pb], 0, 0, 0);
+        if (!QF16) sc[pb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka, ql[ss], sc[pb], 0, 0, 0);
       }
-      sc[pb] = acc;
+    __builtin_amdgcn_sched_group_barrier(0x100, kAttnKAhead, 0);  // LDS reads
+#pragma unroll
+    for (int i = 0; i < 16 - kAttnKAhead; i++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, QF16 ? 1 : 2, 0);  // MFMA
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);             // LDS read
     }
+    __builtin_amdgcn_sched_group_barrier(0x008, (QF16 ? 1 : 2) * kAttnKAhead, 0);
     float tmax = -INFINITY;
     if (wave_full && t0 + kAttnTile <= wave_hi) {
 #pragma unroll
@@ -638,6 +653,14 @@ __device__ __forceinline__ void attn_prefill(const AttnArgs& a, const AttnItem& 
           if (!QF16) o[db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pfl[pb][t], o[db], 0, 0, 0);
         }
       }
+    // V fragments (two reads each) kAttnVAhead ahead of their MFMAs likewise
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kAttnVAhead, 0);  // LDS reads
+#pragma unroll
+    for (int i = 0; i < 16 - kAttnVAhead; i++) {
+      __builtin_amdgcn_sched_group_barrier(0x008, QF16 ? 1 : 2, 0);  // MFMA
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);             // LDS reads
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, (QF16 ? 1 : 2) * kAttnVAhead, 0);
   }
 
   if (!valid) return;
@@ -837,10 +860,15 @@ int attn_build_plan(int T, int B, const uint32_t* lengths, const uint32_t* exten
     return fail(TGOHIP_EINVAL, "attention: the extents sum to " + std::to_string(at) +
                                    " and q has " + std::to_string(T) + " rows");
   plan.claimed = (int)at;
-  // Positions per part of a context-split item (multiples of the 64-position
-  // tile). Decode-style items stream: long parts amortize a workgroup's start
-  // (page staging, first loads) and merge. Prefill-style items are MFMA-bound:
-  // shorter parts spread a chunk's work over more workgroups. Both depend only
+  // Most positions per part of a context-split item (multiples of the 64-position
+  // tile). Decode-style items stream, and long parts amortize a workgroup's start
+  // (page staging, first loads) and merge; prefill-style items write 64 KiB of
+  // sums per part. Equal parts keep the launch's longest item short. Measured,
+  // equal parts, decode / prefill 2560 / 2048, 2560 / 3072, 2560 / 4096, 2048 /
+  // 2048 (us): 128 decodes 198.5, 198.3, 198.5, 195.3; 8 chunks of 256 beside 56
+  // decodes 199.7, 193.4, 241.5, 197.6; four chunks of 512, f16 q, 122.2, 120.7,
+  // 114.5, 122.0; with full parts and a remainder at 2560 / 2048: 201.1, 197.7,
+  // 126.0. Both depend only
   // on the sequence itself, so a mixed launch decomposes every sequence as it
   // would alone. TGOHIP_ATTN_SPLIT / TGOHIP_ATTN_PSPLIT override them.
   // An override is capped so that a part's page-16 table always fits the
@@ -856,6 +884,11 @@ int attn_build_plan(int T, int B, const uint32_t* lengths, const uint32_t* exten
     const int v = std::min(e ? atoi(e) : kAttnSplitPrefill, kSplitCap);
     return v >= kAttnTile ? v / kAttnTile * kAttnTile : kAttnSplitPrefill;
   }();
+  // Positions per part when `len` go into `parts`: equal parts of whole tiles,
+  // not full ones and a remainder, so that the longest item of a launch is short.
+  auto even_part = [](int len, int parts) {
+    return ((len + parts - 1) / parts + kAttnTile - 1) / kAttnTile * kAttnTile;
+  };
   // Shared prefixes (opt-in): decode sequences (one token) whose page rows
   // begin with the same pages attend to those positions together. A group's
   // prefix is the longest run of pages every member shares, cut to whole
@@ -984,9 +1017,9 @@ int attn_build_plan(int T, int B, const uint32_t* lengths, const uint32_t* exten
         for (int kvh = 0; kvh < Hkv; kvh++)
           plan.items.push_back(AttnItem{s, kvh, 0, n, 0, L, -1, dmode(s, 0)});
       } else {
-        const int base = plan.parts;
+        const int base = plan.parts, step = even_part(L, splits);
         for (int p = 0; p < splits; p++) {
-          const int lo = p * split, hi = std::min(L, lo + split);
+          const int lo = p * step, hi = std::min(L, lo + step);
           for (int kvh = 0; kvh < Hkv; kvh++)
             plan.items.push_back(AttnItem{s, kvh, 0, n, lo, hi, base + kvh * splits + p, dmode(s, lo)});
         }
@@ -1007,8 +1040,9 @@ int attn_build_plan(int T, int B, const uint32_t* lengths, const uint32_t* exten
             plan.items.push_back(AttnItem{s, kvh, t0, nt, 0, hi, -1, 1});
           } else {
             const int part0 = plan.parts;
+            const int step = even_part(hi, splits);
             for (int p = 0; p < splits; p++) {
-              const int lo = p * psplit, h2 = std::min(hi, lo + psplit);
+              const int lo = p * step, h2 = std::min(hi, lo + step);
               plan.items.push_back(AttnItem{s, kvh, t0, nt, lo, h2, plan.parts++, 1});
             }
             plan.combines.push_back(AttnCombine{s, kvh, t0, nt, part0, splits, -1, 0, 0, 0});
