@@ -119,6 +119,8 @@ struct Layer {
 
 using namespace tgohip;
 
+constexpr int kPinnedSlots = 4;
+
 struct tgohip_ctx {
   int device = 0;
   hipStream_t own_stream = nullptr;
@@ -148,10 +150,15 @@ struct tgohip_ctx {
   // The head of the last launched step ran over the members that worked only:
   // logits row i is member head_rows[i]'s (empty: one row per member).
   std::vector<int32_t> head_rows;
-  // pinned staging for per-step metadata
-  void* pinned = nullptr;
-  size_t pinned_bytes = 0;
-  hipEvent_t staged = nullptr;  // the last H2D copy out of `pinned`
+  // pinned staging for per-call metadata: a call writes the next slot while the
+  // device still reads the ones before, and waits only for the slot it takes
+  struct Pinned {
+    void* p = nullptr;
+    size_t bytes = 0;
+    hipEvent_t read = nullptr;  // the device's last read of it
+  };
+  Pinned pinned[kPinnedSlots];
+  int pinned_next = 0;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   std::vector<void*> allocs;  // weight and gain allocations owned by the context
   std::map<int, PackedWeight> handles;
@@ -186,19 +193,24 @@ void free_owned(tgohip_ctx* c, void* p) {
   (void)hipFree(p);
 }
 
-int ensure_pinned(tgohip_ctx* c, size_t bytes) {
-  if (c->staged) TGOHIP_HIP(hipEventSynchronize(c->staged));
-  if (bytes <= c->pinned_bytes) return 0;
-  if (c->pinned) (void)hipHostFree(c->pinned);
-  c->pinned = nullptr;
-  c->pinned_bytes = 0;
-  TGOHIP_HIP(hipHostMalloc(&c->pinned, bytes, hipHostMallocDefault));
-  c->pinned_bytes = bytes;
+// The next staging slot, free and of at least `bytes`.
+int take_pinned(tgohip_ctx* c, size_t bytes, tgohip_ctx::Pinned** out) {
+  tgohip_ctx::Pinned& s = c->pinned[c->pinned_next];
+  c->pinned_next = (c->pinned_next + 1) % kPinnedSlots;
+  TGOHIP_HIP(hipEventSynchronize(s.read));
+  if (bytes > s.bytes) {
+    if (s.p) (void)hipHostFree(s.p);
+    s.p = nullptr;
+    s.bytes = 0;
+    TGOHIP_HIP(hipHostMalloc(&s.p, bytes, hipHostMallocDefault));
+    s.bytes = bytes;
+  }
+  *out = &s;
   return 0;
 }
 
-// Metadata packer: appends arrays into the pinned staging buffer at 256-byte
-// aligned offsets, then one H2D copy moves all of them into c->meta.
+// Metadata packer: appends arrays into a pinned staging slot at 256-byte
+// aligned offsets, then one kernel reads all of them into c->meta.
 struct Stager {
   std::vector<std::pair<const void*, size_t>> parts;
   std::vector<size_t> offs;
@@ -212,14 +224,16 @@ struct Stager {
   }
   int upload(tgohip_ctx* c) {
     if (total == 0) return 0;
-    int rc = ensure_pinned(c, total);
+    tgohip_ctx::Pinned* s = nullptr;
+    int rc = take_pinned(c, total, &s);
     if (rc) return rc;
     rc = c->meta.ensure(total);
     if (rc) return rc;
     for (size_t i = 0; i < parts.size(); i++)
-      if (parts[i].second) memcpy((char*)c->pinned + offs[i], parts[i].first, parts[i].second);
-    TGOHIP_HIP(hipMemcpyAsync(c->meta.p, c->pinned, total, hipMemcpyHostToDevice, c->stream));
-    TGOHIP_HIP(hipEventRecord(c->staged, c->stream));
+      if (parts[i].second) memcpy((char*)s->p + offs[i], parts[i].first, parts[i].second);
+    launch_fetch(s->p, c->meta.p, total, c->stream);
+    TGOHIP_HIP(hipGetLastError());
+    TGOHIP_HIP(hipEventRecord(s->read, c->stream));
     return 0;
   }
   template <class T> T* dev(tgohip_ctx* c, size_t off) { return (T*)((char*)c->meta.p + off); }
@@ -550,13 +564,18 @@ tgohip_ctx* tgohip_open(int device) {
   c->ncu = prop.multiProcessorCount;
   c->scratch = scr;
   if (hipStreamCreate(&c->own_stream) != hipSuccess ||
-      hipEventCreateWithFlags(&c->staged, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&c->ev0, hipEventDisableSystemFence) != hipSuccess ||
       hipEventCreate(&c->ev1) != hipSuccess) {
     fail(TGOHIP_EDEVICE, "tgohip_open: stream/event creation failed");
     delete c;
     return nullptr;
   }
+  for (tgohip_ctx::Pinned& p : c->pinned)
+    if (hipEventCreateWithFlags(&p.read, hipEventDisableTiming) != hipSuccess) {
+      fail(TGOHIP_EDEVICE, "tgohip_open: event creation failed");
+      delete c;
+      return nullptr;
+    }
   c->stream = c->own_stream;
   return c;
 }
@@ -573,9 +592,11 @@ void tgohip_close(tgohip_ctx* c) {
     b->release();
   if (c->kc) (void)hipFree(c->kc);
   if (c->vc) (void)hipFree(c->vc);
-  if (c->pinned) (void)hipHostFree(c->pinned);
+  for (tgohip_ctx::Pinned& p : c->pinned) {
+    if (p.p) (void)hipHostFree(p.p);
+    (void)hipEventDestroy(p.read);
+  }
   for (hipEvent_t e : c->prof_ev) (void)hipEventDestroy(e);
-  (void)hipEventDestroy(c->staged);
   (void)hipEventDestroy(c->ev0);
   (void)hipEventDestroy(c->ev1);
   (void)hipStreamDestroy(c->own_stream);
