@@ -791,7 +791,63 @@ __global__ __launch_bounds__((64 * NW * KQ), (8 / (NW * KQ))) void gemm_pipe_ker
                   });
     }
   } else {
-    gemm_epilogue<EPI, MB>(g, acc, m0, nbw0, nbv, h, c32, nsplit > 1, split);
+    // Each wave turns its sums through 8 KiB of the ring, 32 rows x 64 columns at
+    // a time, so that it stores whole 16-byte pieces of a row instead of single
+    // words (64 stores a wave, 4.1 us of a 128-row projection's 14 to 35): [4096,
+    // 4096] of symmetric int4 at 128 pair rows, 8 splits, 17.6 -> 15.8 us, [12288,
+    // 4096] 35.4 -> 33.5, [4096, 24576] at 1152 rows 406 -> 399; f16 operands 21.3
+    // -> 17.9, 37.7 -> 34.5, 209 -> 205. Every wave is done reading the ring; with two k groups the other
+    // group has ended and this wave alone read its part of it.
+    if constexpr (KQ == 1) __syncthreads();
+    const int wst = NW == 8 ? wave >> 1 : wave;
+    float* turn = (float*)(wst == 0 ? As0 : wst == 1 ? As1 : wst == 2 ? As2 : As3) + (NW == 8 ? (wave & 1) * 2048 : 0);
+    constexpr bool SW = EPI == EPI_SWIGLU_F16 || EPI == EPI_SWIGLU_F32 || EPI == EPI_SWIGLU_X2;
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++) {
+      // row r's columns 0-31 and 32-63 trade places where r & 4, so that the two
+      // rows of a store sit in different banks
+#pragma unroll
+      for (int b = 0; b < 2; b++)
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+          turn[(8 * (r >> 2) + 4 * h + (r & 3)) * 64 + ((b ^ h) * 32 + c32)] = acc[mb][b][r];
+      __builtin_amdgcn_wave_barrier();
+      const int m1 = m0 + mb * 32;
+      if (SW && nsplit <= 1) {
+        if (nbv[1]) {
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int row = 8 * i + (lane >> 3), c4 = (lane & 7) * 4, f = ((row >> 2) & 1) * 32;
+            if (m1 + row >= g.M) continue;
+            const float4_t ga = *(const float4_t*)(turn + row * 64 + (c4 ^ f));
+            const float4_t ua = *(const float4_t*)(turn + row * 64 + ((c4 + 32) ^ f));
+            const size_t o = (size_t)(m1 + row) * (g.N / 2) + (nbw0 >> 1) * 32 + c4;
+            store_swiglu4<EPI>(g, o, ga, ua);
+          }
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          const int row = 4 * i + (lane >> 4), c4 = (lane & 15) * 4;
+          if (m1 + row >= g.M || !nbv[c4 >> 5]) continue;
+          const float4_t v = *(const float4_t*)(turn + row * 64 + (c4 ^ ((i & 1) * 32)));
+          const size_t o = (size_t)(m1 + row) * g.N + (size_t)nbw0 * 32 + c4;
+          if (nsplit > 1) {
+            *(float4_t*)(g.part + (size_t)split * g.pstride + o) = v;
+          } else if (EPI == EPI_F16) {
+            *(half4_t*)((half_t*)g.y + o) = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+          } else if (EPI == EPI_RESID) {
+            float4_t y = *(const float4_t*)((float*)g.y + o);
+#pragma unroll
+            for (int e = 0; e < 4; e++) y[e] += v[e];
+            *(float4_t*)((float*)g.y + o) = y;
+          } else {
+            *(float4_t*)((float*)g.y + o) = v;
+          }
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
   }
 #undef PIPE_DMA_A
 }

@@ -313,6 +313,26 @@ __device__ __forceinline__ void store_swiglu(const GemmArgs& g, size_t o, float 
   }
 }
 
+// Four consecutive SwiGLU outputs at element o (store_swiglu's values).
+template <int EPI>
+__device__ __forceinline__ void store_swiglu4(const GemmArgs& g, size_t o, float4_t gate, float4_t up) {
+  float4_t v;
+#pragma unroll
+  for (int e = 0; e < 4; e++) v[e] = silu_f(gate[e]) * up[e];
+  if (EPI == EPI_SWIGLU_F32) {
+    *(float4_t*)((float*)g.y + o) = v;
+    return;
+  }
+  half4_t hv, lv;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    hv[e] = (half_t)v[e];
+    lv[e] = (half_t)(v[e] - (float)hv[e]);
+  }
+  *(half4_t*)((half_t*)g.y + o) = hv;
+  if (EPI == EPI_SWIGLU_X2) *(half4_t*)((half_t*)g.y + (size_t)g.M * (g.N / 2) + o) = lv;
+}
+
 // A workgroup barrier that orders LDS only: global loads in flight stay in
 // flight across it (__syncthreads would wait for them).
 __device__ __forceinline__ void lds_barrier() {
