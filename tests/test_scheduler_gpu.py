@@ -81,6 +81,23 @@ def test_derived_ports_equal_the_packed_ports(torch_gpu, rows_pad):
     b.close()
 
 
+def test_per_head_positions_equal_the_row_table(torch_gpu):
+    """Packed ports give a row's heads one position, and the angles come from the step's
+    table. One differing head of the decode's row takes every row to the per-head angles:
+    the other members' logits, which don't see that row, stay equal to the bit."""
+    st, table, max_pages = packed_step(np.random.default_rng(7), 0)
+    for port, heads in (("posq", CFG["heads"]), ("posk", CFG["kv_heads"])):
+        odd = dict(st, **{port: list(st[port])})
+        odd[port][int(st["last"][2]) * heads] += 1
+        a, b = new_ctx(torch_gpu), new_ctx(torch_gpu)
+        la, aa, _ = a.step(st, table, max_pages)
+        lb, ab, _ = b.step(odd, table, max_pages)
+        assert la[0].any() and np.array_equal(la[0], lb[0]) and aa[0] == ab[0]
+        assert np.isfinite(lb).all() and not np.array_equal(la[2], lb[2])
+        a.close()
+        b.close()
+
+
 def test_fused_qkv_epilogue_equals_the_separate_kernel(torch_gpu):
     """69 rows (a 48-token chunk, an idle member, a decode, a 20-token chunk after 10 cached
     positions): the QKV projection runs on the pipelined exact kernel, unsplit with one k

@@ -1022,11 +1022,31 @@ int step_launch(tgohip_ctx* c, const tgohip_batch_step* s, StepLaunch& o) {
   if ((rc = ensure_activations(c, Tw, B, HB))) return rc;
   if ((rc = ensure_attn_parts(c, plan.parts))) return rc;
 
+  // Packed ports (NewBatchStep) give all heads of a row one position: the row's
+  // angles then come from a table made once per step, as derived rows' do,
+  // instead of f64 sin and cos in every layer. Ports that give heads of a row
+  // different positions keep the per-head ones.
+  std::vector<uint32_t> rowpos;
+  if (!derived) {
+    bool same = true;
+    rowpos.resize(Tw);
+    for (int t = 0; t < Tw && same; t++) {
+      const uint32_t p = rowpos[t] = s->posq[(size_t)t * m.heads];
+      uint32_t diff = 0;
+      for (int i = 0; i < m.heads; i++) diff |= s->posq[(size_t)t * m.heads + i] ^ p;
+      for (int i = 0; i < m.kv_heads; i++) diff |= s->posk[(size_t)t * m.kv_heads + i] ^ p;
+      same = diff == 0 && p <= 0x7fffffffu;  // the kernels take it as an int
+    }
+    if (!same) rowpos.clear();
+  }
+  const bool by_row = derived || !rowpos.empty();  // one position per row
+
   // One staged upload of every port (batch.go:385-405).
   Stager sg;
   const size_t o_ids = sg.add(s->ids, (size_t)Tw * 4);
-  const size_t o_posq = derived ? 0 : sg.add(s->posq, (size_t)Tw * m.heads * 4);
-  const size_t o_posk = derived ? 0 : sg.add(s->posk, (size_t)Tw * m.kv_heads * 4);
+  const size_t o_posq = by_row ? 0 : sg.add(s->posq, (size_t)Tw * m.heads * 4);
+  const size_t o_posk = by_row ? 0 : sg.add(s->posk, (size_t)Tw * m.kv_heads * 4);
+  const size_t o_rowpos = rowpos.empty() ? 0 : sg.add(rowpos.data(), (size_t)Tw * 4);
   const size_t o_slots = derived ? 0 : sg.add(s->slots, (size_t)Tw * 4);
   const size_t o_len = sg.add(s->lengths, (size_t)B * 4);
   const size_t o_ext = sg.add(s->extents, (size_t)B * 4);
@@ -1109,8 +1129,10 @@ int step_launch(tgohip_ctx* c, const tgohip_batch_step* s, StepLaunch& o) {
     launch_derive_rows(DeriveArgs{dp.cu, dp.lengths, d_ext, dp.pages, B, s->max_pages, m.block,
                                   plan.claimed, pad, Tw, c->kv_positions, d_rowpos, d_rowslot},
                        st);
-    launch_rope_table(d_rowpos, Tw, c->inv_freq, (float4_t*)c->rope.p, st);
+  } else {
+    d_rowpos = by_row ? sg.dev<uint32_t>(c, o_rowpos) : nullptr;
   }
+  if (by_row) launch_rope_table(d_rowpos, Tw, c->inv_freq, (float4_t*)c->rope.p, st);
   // A split-K projection's partial planes are summed by the kernel that reads
   // its output next (in split order, so the result is the reduction's):
   // QKV's by qk_rope_kv, O's and down's (residual adds) by the following
@@ -1134,12 +1156,12 @@ int step_launch(tgohip_ctx* c, const tgohip_batch_step* s, StepLaunch& o) {
     int qkv_split = 0;
     QKRopeArgs qa{nullptr, 0, split_plane_stride(Tw, (m.heads + 2 * m.kv_heads) * kHeadDim),
                   L.g_q, L.g_k,
-                  derived ? nullptr : sg.dev<uint32_t>(c, o_posq),
-                  derived ? nullptr : sg.dev<uint32_t>(c, o_posk),
-                  derived ? d_rowslot : sg.dev<uint32_t>(c, o_slots), derived ? d_rowpos : nullptr,
+                  by_row ? nullptr : sg.dev<uint32_t>(c, o_posq),
+                  by_row ? nullptr : sg.dev<uint32_t>(c, o_posk),
+                  derived ? d_rowslot : sg.dev<uint32_t>(c, o_slots), d_rowpos,
                   c->inv_freq, c->q.p, c->kc + l * layer_kv,
                   c->vc + l * layer_kv, m.heads, m.kv_heads, c->kv_positions, m.rms_eps, qf16,
-                  derived ? (const float4_t*)c->rope.p : nullptr};
+                  by_row ? (const float4_t*)c->rope.p : nullptr};
     if ((rc = mark(TGOHIP_PROF_QKV, l, 0))) return rc;
     if (fuse_qk) {
       // q/k-norm, RoPE and the K/V write in the projection's epilogue
