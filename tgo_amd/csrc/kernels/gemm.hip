@@ -1797,19 +1797,27 @@ static bool use_pipe(const PackedWeight& w, int xk, int M) {
 //    packs 8192 to 16384 at 4 rows and more: [12288, 4096] at 8 rows 25.9 -> 18.2)
 //    and for a K that leaves that kernel fewer than four waves ([5504, 3584] of
 //    int8 at 2 rows, one wave: 57 us).
-//  * otherwise while all workgroups together read at most 64 MB of activations
-//    (80 above 32 rows): [1024, 6144] pairs at 32 rows (25 MB) 11.6 -> 6.7 and at 67
-//    (53 MB) 17.3 -> 13.6; at 128 (100 MB) 19.1 -> 19.0, and [4096, 6144] at 40
-//    (126 MB) 19.5 -> 28. A launch of under half the CUs splits K from 2048 up
-//    ([4096, 1024] at 67 rows 31.8 -> 13.1; [1024, 1024] 9.6 -> 10.2).
+//  * otherwise while all workgroups together read few activations: over a K of at
+//    most 4096, up to 105 MB of pairs or f32 rows up to 32 ([4096, 6144] of symmetric int4 at 32 pair
+//    rows, 100 MB, 18.1 -> 12.3), above that 140 MB of pairs ([1024, 4096] at 256,
+//    134 MB, 18.4 -> 12.3; [4096, 4096] at 64 18.3 -> 14.4) and 110 of f32 rows
+//    ([1024, 6144] at 128, 100 MB, 19.0 -> 12.9; [4096, 6144] of int8 at 40, 126 MB,
+//    21.9 against 23.2); 64 or 80 MB over a longer K ([8192, 5120] of int8 at 18
+//    pair rows, 94 MB, 21.5 against 26.4) or of f16 operands ([1024, 6144] of int8 at
+//    192, 75 MB, 17.4 -> 13.0). A launch of under half the CUs splits K from 2048
+//    up ([4096, 1024] at 67 rows 31.8 -> 9.9; [1024, 1024] 9.6 -> 10.2). Above 32
+//    rows, f16 weights take two column blocks per workgroup where that makes one
+//    round of two ([1024, 6144] at 67 pair rows 13.1 -> 9.3, with one block 12.2).
 struct RowsShape {
   int cb, splits;
 };
 static RowsShape rows_shape(const PackedWeight& w, int xk, int M, int epi, int ncu) {
   const bool sw = epi == EPI_SWIGLU_F16 || epi == EPI_SWIGLU_X2;
   RowsShape r{0, 1};
-  const int KS = w.K / 64, cb = sw ? 2 : 1;
-  const int groups = (w.N / 32 + cb - 1) / cb * (M > 32 ? (M + 63) / 64 : 1);
+  const int KS = w.K / 64, mt = M > 32 ? (M + 63) / 64 : 1;
+  int cb = sw ? 2 : 1;
+  if (w.form == TGOHIP_FORM_F16 && xk != XK_F32 && M > 32 && w.N / 32 * mt > ncu && (w.N / 32 + 1) / 2 * mt <= ncu) cb = 2;
+  const int groups = (w.N / 32 + cb - 1) / cb * mt;
   // the planes of a split fit the allocation-free linear's array
   auto planes_fit = [&](int s) {
     return s == 1 || (size_t)s * split_plane_stride(M, w.N) * sizeof(float) <= kRowsPlaneBytes;
@@ -1833,7 +1841,8 @@ static RowsShape rows_shape(const PackedWeight& w, int xk, int M, int epi, int n
   const int64_t traffic = (int64_t)(w.N / 32 + cb - 1) / cb * M * w.K * (xk == XK_F16 ? 2 : 4);
   // half of that where a second round of workgroups would be mostly empty
   // ([5120, 10240] at 16 f16 rows, 320 column blocks, 52 MB: 27.0 us against 29.1)
-  const int64_t most = (int64_t)(groups > ncu && groups < 2 * ncu && M <= 32 ? 40 : M <= 32 ? 64 : 80) * 1000000;
+  const int64_t most = (int64_t)(groups > ncu && groups < 2 * ncu && M <= 32 ? 40 : M <= 32 ? (xk == XK_F16 || KS > 64 ? 64 : 105)
+                                              : (xk == XK_F16 || KS > 64 ? 80 : xk == XK_X2 ? 140 : 110)) * 1000000;
   if (traffic > most) return r;
   r.cb = cb;
   if (KS >= 32)

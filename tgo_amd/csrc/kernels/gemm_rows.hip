@@ -4,8 +4,8 @@
 //
 // A workgroup of 8 or 16 waves owns 32 * CB columns and 32 * MB rows. The waves take
 // the k-steps (64 deep) of its share of K in turn, each with its own weight
-// fragments (registers, two k-steps ahead) and activation fragments (read from
-// L2 as MFMA operands, one k-step ahead), and meet once, in LDS, where their
+// fragments (registers, two k-steps ahead) and activations (one k-step ahead),
+// and meet once, in LDS, where their
 // sums are added in wave order: one barrier per launch instead of one per
 // k-step, and 8 waves' loads in flight on each CU from the first cycle.
 #include "gemm_weights.h"
@@ -46,11 +46,15 @@ __device__ __forceinline__ int rows_chunk(int r, int c) { return c ^ (r & 7); }
 // lane and are added at the end.
 // STG (PACK only): the workgroup's share of the activations goes to LDS once,
 // split into hi and lo there, after the first weight loads are issued; the
-// weight stream is then the only vector-memory traffic of the loop. Without
-// it a wave reads its A operands from L2 (every load touches a cache line per
-// row), and f32 rows are split again by every lane that repeats one.
-template <int FORM, int XK, int MB, int CB, bool PACK, bool STG, int W>
-__global__ __launch_bounds__(64 * W, W == 16 || (MB * CB == 1 && FORM != TGOHIP_FORM_I4_TGO) ? 4 : 2) void gemm_rows_kernel(
+// weight stream is then the only vector-memory traffic of the loop.
+// TURN: a wave loads its rows of a k-step as whole 128-byte lines, eight lanes
+// each, and turns them into MFMA operands in its own part of LDS. Operands
+// loaded straight from L2 touch a quarter of 32 lines each, and the L1 misses
+// bound the launch: [1024, 4096] of f16 weights at 67 pair rows 10.0 -> 6.8 us,
+// [3072, 1024] 11.2 -> 8.5, [4096, 6144] at 20 rows 20.6 -> 14.4.
+// Neither (PACK, or one k-step per wave): operands from L2.
+template <int FORM, int XK, int MB, int CB, bool PACK, bool STG, int W, bool TURN>
+__global__ __launch_bounds__(64 * W, W == 16 || (MB * CB == 1 && FORM != TGOHIP_FORM_I4_TGO && !(FORM == TGOHIP_FORM_I8 && XK == XK_F32 && TURN)) ? 4 : 2) void gemm_rows_kernel(
     GemmArgs g, int epi) {
   constexpr bool EX = XK != XK_F16;                          // tgo's arithmetic
   constexpr bool FX = EX && FORM == TGOHIP_FORM_I4_SYM;      // factored group scales
@@ -80,10 +84,59 @@ __global__ __launch_bounds__(64 * W, W == 16 || (MB * CB == 1 && FORM != TGOHIP_
   const int sk = nk * 64, sr = min(c32 & 15, g.M - 1);
   const half_t* const srow = (const half_t*)smem + (size_t)((lolane ? g.M : 0) + sr) * sk;
 
+  // TURN: the wave's rows of a k-step, whole 128-byte lines of 8 lanes each, on
+  // their way to its own part of LDS, where they are read as operands.
+  half_t* const turn = (half_t*)smem + (size_t)wave * AP * MB * 2048;
+  const int tc = lane & 7, tr = lane >> 3;
+  uint4 tq[TURN ? 4 * MB : 1][XK == XK_F16 ? 1 : 2];
+  auto load_turn = [&](int ks) {
+    if constexpr (TURN) {
+#pragma unroll
+      for (int t = 0; t < 4 * MB; t++) {
+        const size_t o = (size_t)min(m0 + 8 * t + tr, g.M - 1) * g.K + (size_t)ks * 64 + 8 * tc;
+        if constexpr (XK == XK_F32) {
+          tq[t][0] = *(const uint4*)(xf + o);
+          tq[t][1] = *(const uint4*)(xf + o + 4);
+        } else {
+          tq[t][0] = *(const uint4*)(xh + o);
+          if constexpr (AP == 2) tq[t][AP - 1] = *(const uint4*)(xl + o);
+        }
+      }
+    }
+  };
+  // Only this wave reads what it writes here, and its LDS operations stay in order.
+  auto store_turn = [&] {
+    if constexpr (TURN) {
+#pragma unroll
+      for (int t = 0; t < 4 * MB; t++) {
+        half_t* const dst = turn + (8 * t + tr) * 64 + 8 * rows_chunk(tr, tc);
+        if constexpr (XK == XK_F32) {
+          union { uint4 u[2]; float f[8]; } r;
+          r.u[0] = tq[t][0];
+          r.u[1] = tq[t][1];
+          half8_t hv, lv;
+#pragma unroll
+          for (int e = 0; e < 8; e++) {
+            hv[e] = (half_t)r.f[e];
+            lv[e] = (half_t)(r.f[e] - (float)hv[e]);
+          }
+          *(half8_t*)dst = hv;
+          *(half8_t*)(dst + MB * 2048) = lv;
+        } else {
+          U16B u;
+          u.u = tq[t][0];
+          *(half8_t*)dst = u.h;
+          u.u = tq[t][AP - 1];
+          if constexpr (AP == 2) *(half8_t*)(dst + MB * 2048) = u.h;
+        }
+      }
+    }
+  };
+
   struct ARaw { uint4 v[XK == XK_F32 ? 2 : AP]; };  // f32: eight floats; else hi (and lo)
-  ARaw aq[STG ? 1 : 4][MB];
+  ARaw aq[STG || TURN ? 1 : 4][MB];
   auto load_a = [&](int j, int ks) {
-    if constexpr (!STG) {
+    if constexpr (!STG && !TURN) {
 #pragma unroll
       for (int mb = 0; mb < MB; mb++) {
         const size_t o = arow[mb] + (size_t)ks * 64 + 16 * j;
@@ -101,6 +154,13 @@ __global__ __launch_bounds__(64 * W, W == 16 || (MB * CB == 1 && FORM != TGOHIP_
   auto operand = [&](int j, int ks, half8_t(&ah)[MB], half8_t(&al)[MB]) {
     if constexpr (STG) {
       ah[0] = *(const half8_t*)(srow + (ks - k0) * 64 + 8 * rows_chunk(sr, 2 * j + h));
+    } else if constexpr (TURN) {
+#pragma unroll
+      for (int mb = 0; mb < MB; mb++) {
+        const half_t* const src = turn + (mb * 32 + c32) * 64 + 8 * rows_chunk(c32, 2 * j + h);
+        ah[mb] = *(const half8_t*)src;
+        if constexpr (AP == 2) al[mb] = *(const half8_t*)(src + MB * 2048);
+      }
     } else {
 #pragma unroll
       for (int mb = 0; mb < MB; mb++) {
@@ -151,6 +211,7 @@ __global__ __launch_bounds__(64 * W, W == 16 || (MB * CB == 1 && FORM != TGOHIP_
       if (d < n) load_b(d, ks0 + W * d);
     });
   };
+  if (TURN && n > 0) load_turn(ks0);
   first_b();
   if constexpr (STG) {
     // eight elements at a time, four loads of them in flight
@@ -195,7 +256,7 @@ __global__ __launch_bounds__(64 * W, W == 16 || (MB * CB == 1 && FORM != TGOHIP_
       }
     }
     lds_barrier();
-  } else if (n > 0) {
+  } else if (!TURN && n > 0) {
 #pragma unroll
     for (int j = 0; j < 4; j++) load_a(j, ks0);
   }
@@ -208,6 +269,8 @@ __global__ __launch_bounds__(64 * W, W == 16 || (MB * CB == 1 && FORM != TGOHIP_
     constexpr bool MAIN = decltype(mainc)::value;
     const int ks = ks0 + W * i;
     float16_t accg[FX ? MB : 1][CB];
+    store_turn();
+    if (MAIN || i + 1 < n) load_turn(ks + W);
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       half8_t ah[MB], al[MB];
@@ -280,7 +343,7 @@ __global__ __launch_bounds__(64 * W, W == 16 || (MB * CB == 1 && FORM != TGOHIP_
 
     // The waves' sums, [rows][32] per column block: lane (c32, h) holds rows
     // 8 (r/4) + 4 h + r%4 of each 32 x 32 block.
-    if constexpr (STG) lds_barrier();  // the sums before have been read
+    if constexpr (STG || TURN) lds_barrier();  // the sums before, or the rows, have been read
 #pragma unroll
     for (int b = 0; b < CB; b++)
 #pragma unroll
@@ -334,21 +397,22 @@ bool rows_staged(int M, int ksteps) {
   return M <= 16 && rows_stage_bytes(M, ksteps) + rows_sum_bytes(M) <= kRowsLdsMax;
 }
 
-template <int FORM, int XK, int MB, int CB, bool PACK, bool STG, int W>
+template <int FORM, int XK, int MB, int CB, bool PACK, bool STG, int W, bool TURN = false>
 static void launch_rows_one(const GemmArgs& g, int epi, int splits, hipStream_t st) {
   const int groups = (g.N / 32 + CB - 1) / CB;
   dim3 grid((unsigned)groups, (unsigned)((g.M + 32 * MB - 1) / (32 * MB)), (unsigned)splits);
-  size_t lds = (size_t)W * MB * CB * 4096;
+  // the waves' sums, or the rows they turn
+  size_t lds = (size_t)W * MB * std::max(CB, TURN && XK != XK_F16 ? 2 : 1) * 4096;
   if (STG) {
     lds = (size_t)(rows_stage_bytes(g.M, g.ksteps_per_split) + rows_sum_bytes(g.M));
     // one workgroup per CU (16 waves of up to 128 registers), each over every
     // 256th column group
     grid.x = (unsigned)std::min(groups, std::max(1, kRowsPersist / splits));
   }
-  static const hipError_t attr = hipFuncSetAttribute((const void*)&gemm_rows_kernel<FORM, XK, MB, CB, PACK, STG, W>,
+  static const hipError_t attr = hipFuncSetAttribute((const void*)&gemm_rows_kernel<FORM, XK, MB, CB, PACK, STG, W, TURN>,
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, kRowsLdsMax);
   (void)attr;
-  hipLaunchKernelGGL((gemm_rows_kernel<FORM, XK, MB, CB, PACK, STG, W>), grid, dim3(64 * W), lds, st, g, epi);
+  hipLaunchKernelGGL((gemm_rows_kernel<FORM, XK, MB, CB, PACK, STG, W, TURN>), grid, dim3(64 * W), lds, st, g, epi);
 }
 
 template <int FORM, int XK, int MB, int CB>
@@ -358,7 +422,12 @@ static void launch_rows_cb(const GemmArgs& g, int epi, int splits, hipStream_t s
       return launch_rows_one<FORM, XK, 1, CB, true, true, CB == 1 ? 16 : 8>(g, epi, splits, st);
     if (g.M <= 16) return launch_rows_one<FORM, XK, 1, CB, true, false, 8>(g, epi, splits, st);
   }
-  launch_rows_one<FORM, XK, MB, CB, false, false, 8>(g, epi, splits, st);
+  // One k-step a wave over one row block: its operands straight from L2, without
+  // the way through LDS ([2048, 1024] of f16 weights at 32 pair rows 7.2 us
+  // against 8.2).
+  if constexpr (MB == 1)
+    if (g.ksteps_per_split <= 8) return launch_rows_one<FORM, XK, MB, CB, false, false, 8>(g, epi, splits, st);
+  launch_rows_one<FORM, XK, MB, CB, false, false, 8, true>(g, epi, splits, st);
 }
 
 template <int FORM>
