@@ -80,6 +80,18 @@ def test_linear_over_few_rows(ctx, torch_gpu, form, K, N, M, xk):
     check(torch_gpu, ctx, form, K, N, M, xk, 11 + K + M)
 
 
+@pytest.mark.parametrize("xk", ["f32", "x2", "f16"])
+@pytest.mark.parametrize("form", [0, 1, 2, 3])
+@pytest.mark.parametrize("K,N,M", [
+    (320, 4224, 65),    # two row tiles of 132 column blocks: f16 weights pair the blocks
+    (1088, 8192, 128),  # 17 k-steps over 8 waves, the pair of blocks at its largest
+    (576, 128, 32), (512, 128, 33),  # just past and at one k-step a wave, one and two row blocks
+    (4096, 2048, 48),   # split K, whole lines of every wave
+])
+def test_linear_turns_its_rows_in_lds(ctx, torch_gpu, form, K, N, M, xk):
+    check(torch_gpu, ctx, form, K, N, M, xk, 11 + K + M)
+
+
 @pytest.mark.parametrize("form", [0, 1, 2, 3])
 @pytest.mark.parametrize("K,N,M", [(4096, 4096, 4200), (4096, 4096, 257)])
 def test_f32_activations_in_bands(ctx, torch_gpu, form, K, N, M):
