@@ -269,6 +269,22 @@ int tgohip_linear_noalloc(tgohip_ctx* ctx, int handle, const void* x, int x_dtyp
  * may go in bands, with the same result). */
 int tgohip_linear_workspace(tgohip_ctx* ctx, int handle, int x_dtype, int M, size_t* bytes);
 
+/* What a projection of M rows by a [K,N] weight of `form` runs on a GPU of
+ * `ncu` compute units: the library's dispatch rules, without a device. No
+ * counterpart in the reference. epilogue: 0 f32, 1 f16, 2 residual add, 3
+ * SwiGLU to f16, 4 to f32, 5 to an activation pair. */
+#define TGOHIP_LINEAR_ROWS 0  /* all of K per workgroup, waves taking its steps in turn */
+#define TGOHIP_LINEAR_PIPE 1  /* the pipelined kernel */
+#define TGOHIP_LINEAR_GEMV 2  /* up to 32 f16 rows */
+#define TGOHIP_LINEAR_TILES 3 /* the tiled kernel */
+typedef struct {
+  int32_t kernel, splits, column_blocks; /* column_blocks: per workgroup (ROWS) */
+  size_t array_bytes; /* what tgohip_linear_noalloc writes in its array */
+  size_t limit_bytes; /* the bytes it takes or refuses the call by */
+} tgohip_linear_plan_t;
+int tgohip_linear_plan(int form, int K, int N, int x_dtype, int M, int epilogue, int ncu,
+                       tgohip_linear_plan_t* plan);
+
 /* Dequantizes a handle's weight to f32 [K,N] on the device exactly as the
  * host restatement does ((q - z) * s in f32). y: device [K,N] f32. */
 int tgohip_dequant(tgohip_ctx* ctx, int handle, float* y);

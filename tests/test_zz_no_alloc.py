@@ -51,6 +51,37 @@ def test_noalloc_linear_equals_linear(ctx, torch_gpu, form, K, N, Ms, xf):
         ctx.weight_free(h)
 
 
+@pytest.mark.parametrize("form,K,N,M", [
+    (tgo_amd.FORM_F16, 1024, 151936, 60),      # 2 planes of 36 MiB: bands of 55 and 5 rows
+    (tgo_amd.FORM_F16, 2048, 51200, 100),      # 4 planes of 20 MiB: a 64-row tile and 36 rows
+    (tgo_amd.FORM_I8, 1600, 65536, 150),       # 25 k-steps, no whole number of groups of four
+    (tgo_amd.FORM_I4_TGO, 1600, 51200, 110),
+    (tgo_amd.FORM_I4_SYM, 1600, 49152, 120),
+])
+def test_noalloc_pairs_go_in_bands_where_their_planes_exceed_the_array(ctx, torch_gpu, form, K, N, M):
+    """Activation pairs whose split-K planes take more than the array while the call's limit
+    does not: the rows go in bands, with tgohip_linear's result to the bit."""
+    torch = torch_gpu
+    p = tgo_amd.linear_plan(form, K, N, tgo_amd.F16X2, M)
+    assert p.splits * M * N * 4 > 64 << 20 >= p.limit_bytes
+    h = weight(ctx, form, K, N, 31 + form)
+    try:
+        print("no-alloc bands: form %d [%d,%d] M=%d" % (form, K, N, M), flush=True)
+        x = torch.randn(M, K, device="cuda", generator=torch.Generator(device="cuda").manual_seed(M))
+        hi = x.half()
+        x = torch.stack([hi, (x - hi.float()).half()])
+        for dt, yd in ((torch.float32, tgo_amd.F32), (torch.float16, tgo_amd.F16)):
+            want = torch.full((M, N), float("nan"), device="cuda", dtype=dt)
+            got = torch.full((M, N), float("nan"), device="cuda", dtype=dt)
+            ctx.linear(h, x, M, want, x_dtype=tgo_amd.F16X2, y_dtype=yd)
+            ctx.linear_noalloc(h, x, M, got, x_dtype=tgo_amd.F16X2, y_dtype=yd)
+            torch.cuda.synchronize()
+            assert torch.isfinite(want).all()
+            assert torch.equal(got, want)
+    finally:
+        ctx.weight_free(h)
+
+
 def test_noalloc_linear_refuses_beyond_its_workspace(ctx, torch_gpu):
     """f32 activations over [12288, 4096] at M = 2100: two partial planes of 34 MiB."""
     torch = torch_gpu

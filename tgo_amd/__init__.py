@@ -16,6 +16,7 @@ LIB_PATH = os.path.join(HERE, "libtgohip.so")
 
 FORM_F16, FORM_I8, FORM_I4_TGO, FORM_I4_SYM = 0, 1, 2, 3
 F32, F16, F16X2 = 0, 1, 2
+LINEAR_ROWS, LINEAR_PIPE, LINEAR_GEMV, LINEAR_TILES = range(4)  # LinearPlan.kernel
 PROF_ATTN, PROF_QKV, PROF_O, PROF_GATEUP, PROF_DOWN, PROF_LMHEAD = range(6)
 PROF_NAMES = ("attention", "qkv", "o", "gateup", "down", "lm_head")
 
@@ -41,6 +42,11 @@ class BatchStepC(ctypes.Structure):
                 ("max_pages", ctypes.c_int32)] + [
         (n, ctypes.c_void_p) for n in ("ids", "posq", "posk", "slots", "lengths", "extents",
                                        "last", "pages")]
+
+
+class LinearPlan(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int32) for n in ("kernel", "splits", "column_blocks")] + [
+        (n, ctypes.c_size_t) for n in ("array_bytes", "limit_bytes")]
 
 
 class Timings(ctypes.Structure):
@@ -88,6 +94,7 @@ def lib():
         "tgohip_linear": (I, [P, I, P, I, I, P, I]),
         "tgohip_linear_noalloc": (I, [P, I, P, I, I, P, I]),
         "tgohip_linear_workspace": (I, [P, I, I, I, P]),
+        "tgohip_linear_plan": (I, [I, I, I, I, I, I, I, ctypes.POINTER(LinearPlan)]),
         "tgohip_dequant": (I, [P, I, P]),
         "tgohip_dequant_f16": (I, [P, I, P]),
         "tgohip_greedy": (I, [P, P, I, I, P, P]),
@@ -232,6 +239,13 @@ def victim(live, prompt_len, prefilled, arrived):
     return lib().tgohip_victim(n, ptr(i32(live or [0])), ptr(i32(prompt_len or [0])),
                                ptr(i32(prefilled or [0])),
                                ptr(np.ascontiguousarray(np.asarray(arrived or [0], np.uint64))))
+
+
+def linear_plan(form, K, N, x_dtype, M, epilogue=0, ncu=256):
+    """What a projection runs (LinearPlan), by the library's dispatch rules alone: no GPU."""
+    p = LinearPlan()
+    check(lib().tgohip_linear_plan(form, K, N, x_dtype, M, epilogue, ncu, ctypes.byref(p)))
+    return p
 
 
 def sha256(data: bytes):

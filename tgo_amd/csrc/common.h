@@ -121,6 +121,12 @@ size_t gemm_workspace_bytes(const PackedWeight& w, int M, int ncu);
 // The split-K bytes by which linear_noalloc takes or refuses a call over
 // activations of kind xk with an f32 or f16 epilogue.
 size_t gemm_limit_bytes(const PackedWeight& w, int M, int ncu, int xk);
+// The workspace bytes such a call writes when it is given `cap` of them: its
+// split-K planes and the pair f32 rows are split into, or those of its largest
+// band of rows.
+size_t gemm_call_bytes(const PackedWeight& w, int M, int ncu, int xk, size_t cap);
+// The route of a call over M >= 1 rows and these bytes (tgohip_linear_plan).
+void gemm_plan(const PackedWeight& w, int M, int ncu, int xk, int epi, size_t cap, tgohip_linear_plan_t* out);
 // Workspace bytes for a call over f32 activations that are split into a pair
 // first (0: the call splits them as it reads them). A smaller workspace makes
 // the call go in bands of rows, with the same sums.

@@ -1759,7 +1759,7 @@ static int pipe_min_rows() {
 
 // The pipelined kernel serves f16 activations and activation pairs (XK_X2, the
 // exact kernel); an f32 activation is split into a pair first
-// (gemm_enqueue_f32).
+// (gemm_pipe_bands).
 static bool use_pipe(const PackedWeight& w, int xk, int M) {
   // f16 operands over f16 weights keep gemm_kernel's 128-row tiles where these
   // fill the chip or K is long: [4096, 24576] at 1100 rows 260 us against 297,
@@ -1851,9 +1851,11 @@ static RowsShape rows_shape(const PackedWeight& w, int xk, int M, int epi, int n
   return r;
 }
 
-// Bytes of split-K planes that linear_noalloc's limit applies to: the splits
-// of gemm_kernel's and the pipelined kernel's tiles, none on the small-M
-// kernel. What the call itself writes is no more than this or the limit.
+// Bytes of split-K planes by which linear_noalloc takes or refuses a call: the
+// planes of the kernels that ran such calls before f16 weights, f32 rows and
+// any whole k-step went to the pipelined kernel, kept so that the calls taken
+// and refused stay the same ones. What a call writes (gemm_call_bytes) does not
+// depend on it: a call that is taken always fits, in bands of rows if need be.
 size_t gemm_limit_bytes(const PackedWeight& w, int M, int ncu, int xk) {
   if (M <= 0) return 0;  // nothing launches (and no tiles to divide the slots by)
   int s;
@@ -1916,20 +1918,22 @@ __global__ __launch_bounds__(256) void split_pair_kernel(const float* x, half_t*
 // in every workgroup, takes three MFMAs per product for symmetric int4 too and
 // spills 76-211 VGPRs with 128-row tiles of the other packs ([4096, 12288] of
 // tgo's int4 over 353 f32 rows: 541 us before). The pair and the split-K planes
-// share the workspace; where they don't fit, the rows go in bands, each with
-// the whole call's tile shape and splits, so the bands don't change the sums.
-static size_t f32_band_bytes(const PackedWeight& w, const PipeLaunch& pl, int rows) {
+// share the workspace.
+// Where they don't fit (the allocation-free linear's array), the rows go in
+// bands, each with the whole call's tile shape and splits, so the bands don't
+// change the sums; so do an activation pair's or f16 rows whose planes don't.
+static size_t pipe_band_bytes(const PackedWeight& w, const PipeLaunch& pl, int xk, int rows) {
   const size_t planes = pl.splits > 1 ? (size_t)pl.splits * split_plane_stride(rows, w.N) * sizeof(float) : 0;
-  return planes + (size_t)rows * w.K * sizeof(float);
+  return planes + (xk == XK_F32 ? (size_t)rows * w.K * sizeof(float) : 0);
 }
 // The most rows, up to M, whose band fits `bytes`: whole row tiles, or fewer
 // rows than one tile; 0 when not even one row fits.
-static int f32_band_rows(const PackedWeight& w, const PipeLaunch& pl, int M, size_t bytes) {
-  if (f32_band_bytes(w, pl, M) <= bytes) return M;
+static int pipe_band_rows(const PackedWeight& w, const PipeLaunch& pl, int xk, int M, size_t bytes) {
+  if (pipe_band_bytes(w, pl, xk, M) <= bytes) return M;
   int lo = 0, hi = M;  // band_bytes grows with the rows
   while (hi - lo > 1) {
     const int mid = lo + (hi - lo) / 2;
-    if (f32_band_bytes(w, pl, mid) <= bytes) lo = mid;
+    if (pipe_band_bytes(w, pl, xk, mid) <= bytes) lo = mid;
     else hi = mid;
   }
   return lo >= pl.mw ? lo / pl.mw * pl.mw : lo;
@@ -1939,25 +1943,88 @@ size_t gemm_f32_workspace_bytes(const PackedWeight& w, int M, int ncu) {
   if (M <= 0 || !use_pipe(w, XK_F32, M)) return 0;
   const PipeLaunch pl = pipe_launch(w, M, ncu, EPI_F32, true);
   const int64_t most = std::max<int64_t>(pl.mw, (int64_t)(kPairBytes / sizeof(float)) / w.K / pl.mw * pl.mw);
-  return f32_band_bytes(w, pl, (int)std::min<int64_t>(M, most));
+  return pipe_band_bytes(w, pl, XK_F32, (int)std::min<int64_t>(M, most));
 }
-static int gemm_enqueue_f32(const PackedWeight& w, const float* x, int M, void* y, int epi,
-                            float* workspace, size_t ws_bytes, int ncu, hipStream_t st) {
-  const PipeLaunch pl = pipe_launch(w, M, ncu, epi, true);
-  const int band = workspace ? f32_band_rows(w, pl, M, ws_bytes) : 0;
-  if (band <= 0) return fail(TGOHIP_ESTATE, "linear: the workspace holds no band of the split activation");
+// The pipelined kernel over all M rows in bands that fit the workspace, with an
+// f32 or f16 epilogue.
+static int gemm_pipe_bands(const PackedWeight& w, const void* x, const void* xlo, int xk, int M, void* y,
+                           int epi, float* workspace, size_t ws_bytes, int ncu, hipStream_t st) {
+  const PipeLaunch pl = pipe_launch(w, M, ncu, epi, xk != XK_F16);
+  const int band = pipe_band_rows(w, pl, xk, M, workspace ? ws_bytes : 0);
+  if (band <= 0) return fail(TGOHIP_ESTATE, "linear: the workspace holds no band of the rows");
   const size_t out = epi == EPI_F16 ? sizeof(half_t) : sizeof(float);
   for (int r0 = 0; r0 < M; r0 += band) {
     const int rows = std::min(band, M - r0);
-    const size_t n = (size_t)rows * w.K, planes = f32_band_bytes(w, pl, rows) - n * sizeof(float);
-    half_t* pair = (half_t*)((char*)workspace + planes);
-    hipLaunchKernelGGL(split_pair_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, st,
-                       x + (size_t)r0 * w.K, pair, n);
-    const int rc = gemm_pipe_enqueue(w, pair, pair + n, rows, (char*)y + (size_t)r0 * w.N * out, epi,
-                                     workspace, planes, ncu, st, nullptr, nullptr, M);
+    const size_t n = (size_t)rows * w.K, at = (size_t)r0 * w.K;
+    const size_t planes = pipe_band_bytes(w, pl, XK_X2, rows);
+    const half_t *hi = (const half_t*)x + at, *lo = xlo ? (const half_t*)xlo + at : nullptr;
+    if (xk == XK_F32) {
+      half_t* pair = (half_t*)((char*)workspace + planes);
+      hipLaunchKernelGGL(split_pair_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, st,
+                         (const float*)x + at, pair, n);
+      hi = pair;
+      lo = pair + n;
+    }
+    const int rc = gemm_pipe_enqueue(w, hi, lo, rows, (char*)y + (size_t)r0 * w.N * out, epi, workspace,
+                                     planes, ncu, st, nullptr, nullptr, M);
     if (rc) return rc;
   }
   return 0;
+}
+
+// The kernel a call runs and its split of K: gemm_enqueue launches what this
+// says, and the workspace queries answer from it.
+struct GemmRoute {
+  int kernel;            // TGOHIP_LINEAR_*
+  int splits;            // slices of K: that many planes in the workspace when more than one
+  int ksteps_per_split;  // rows, tiles
+  int cb;                // rows: column blocks per workgroup
+  int mw;                // tiles: rows of a tile
+};
+static GemmRoute gemm_route(const PackedWeight& w, int xk, int M, int epi, int ncu, bool defer) {
+  const int KS = w.K / 64;
+  GemmRoute r{};
+  // A QKV projection (the deferring f32 call) whose derived-rows form fuses its
+  // epilogue keeps the same kernel here, so that both give the same bits.
+  const bool fusable = defer && epi == EPI_F32 && xk == XK_X2 && gemm_qkrope_fusable(w, M, ncu);
+  const RowsShape rs = rows_shape(w, xk, M, epi, ncu);
+  if (rs.cb && !fusable) {
+    r.kernel = TGOHIP_LINEAR_ROWS;
+    r.cb = rs.cb;
+    r.ksteps_per_split = (KS + rs.splits - 1) / rs.splits;
+    r.splits = (KS + r.ksteps_per_split - 1) / r.ksteps_per_split;
+  } else if (use_pipe(w, xk, M) && (xk != XK_F32 || (!defer && (epi == EPI_F32 || epi == EPI_F16)))) {
+    r.kernel = TGOHIP_LINEAR_PIPE;
+    r.splits = pipe_launch(w, M, ncu, epi, xk != XK_F16).splits;
+  } else if (use_gemv(w, xk, M, ncu)) {
+    r.kernel = TGOHIP_LINEAR_GEMV;
+    r.splits = 1;
+  } else {
+    r.kernel = TGOHIP_LINEAR_TILES;
+    r.mw = small_mw(w, M, ncu);
+    r.splits = choose_splits(M, w.N, w.K, r.mw, ncu);
+    r.ksteps_per_split = (KS + r.splits - 1) / r.splits;
+  }
+  return r;
+}
+
+size_t gemm_call_bytes(const PackedWeight& w, int M, int ncu, int xk, size_t cap) {
+  if (M <= 0) return 0;
+  const GemmRoute r = gemm_route(w, xk, M, EPI_F32, ncu, false);
+  if (r.kernel == TGOHIP_LINEAR_PIPE) {
+    const PipeLaunch pl = pipe_launch(w, M, ncu, EPI_F32, xk != XK_F16);
+    return pipe_band_bytes(w, pl, xk, pipe_band_rows(w, pl, xk, M, cap));
+  }
+  return r.splits > 1 ? (size_t)r.splits * split_plane_stride(M, w.N) * sizeof(float) : 0;
+}
+
+void gemm_plan(const PackedWeight& w, int M, int ncu, int xk, int epi, size_t cap, tgohip_linear_plan_t* out) {
+  const GemmRoute r = gemm_route(w, xk, M, epi, ncu, false);
+  out->kernel = r.kernel;
+  out->splits = r.splits;
+  out->column_blocks = r.cb;
+  out->array_bytes = gemm_call_bytes(w, M, ncu, xk, cap);
+  out->limit_bytes = gemm_limit_bytes(w, M, ncu, xk);
 }
 
 int gemm_enqueue(const PackedWeight& w, const void* x, int xk, int M, void* y, int epi,
@@ -1971,62 +2038,12 @@ int gemm_enqueue(const PackedWeight& w, const void* x, int xk, int M, void* y, i
     return fail(TGOHIP_ESTATE, "linear: the activation-pair SwiGLU output goes with activation-pair input");
   // an activation pair's lo plane follows its hi plane
   const void* xlo = xk == XK_X2 ? (const void*)((const half_t*)x + (size_t)M * w.K) : nullptr;
-  // A QKV projection (the deferring f32 call) whose derived-rows form fuses its
-  // epilogue keeps the same kernel here, so that both give the same bits.
-  const bool fusable = defer && epi == EPI_F32 && xk == XK_X2 && gemm_qkrope_fusable(w, M, ncu);
-  const RowsShape rs = rows_shape(w, xk, M, epi, ncu);
-  if (rs.cb && !fusable) {
-    GemmArgs g{};
-    g.x = x;
-    g.xlo = xlo;
-    g.wp = w.wp;
-    g.ws = w.ws;
-    g.wz = w.wz;
-    g.y = y;
-    g.M = M;
-    g.K = w.K;
-    g.N = w.N;
-    g.ksteps_per_split = (w.K / 64 + rs.splits - 1) / rs.splits;
-    const int splits = (w.K / 64 + g.ksteps_per_split - 1) / g.ksteps_per_split;
-    if (splits > 1) {
-      if (!workspace || ws_bytes < (size_t)splits * split_plane_stride(M, w.N) * sizeof(float))
-        return fail(TGOHIP_ESTATE, "linear: split-K workspace too small");
-      g.part = workspace;
-      g.pstride = split_plane_stride(M, w.N);
-    }
-    launch_gemm_rows(w.form, g, xk, epi, rs.cb, splits, st);
-    if (defer) *defer = splits > 1 ? splits : 0;
-    if (splits > 1 && !defer) launch_reduce(g, epi, splits, st);
-    TGOHIP_HIP(hipGetLastError());
-    return 0;
-  }
-  if (xk == XK_F32 && (epi == EPI_F32 || epi == EPI_F16) && !defer && use_pipe(w, xk, M))
-    return gemm_enqueue_f32(w, (const float*)x, M, y, epi, workspace, ws_bytes, ncu, st);
-  if (xk != XK_F32 && use_pipe(w, xk, M))
+  const GemmRoute r = gemm_route(w, xk, M, epi, ncu, defer != nullptr);
+  if (r.kernel == TGOHIP_LINEAR_PIPE) {
+    if ((epi == EPI_F32 || epi == EPI_F16) && !defer)
+      return gemm_pipe_bands(w, x, xlo, xk, M, y, epi, workspace, ws_bytes, ncu, st);
     return gemm_pipe_enqueue(w, x, xlo, M, y, epi, workspace, ws_bytes, ncu, st, defer);
-  if (use_gemv(w, xk, M, ncu)) {
-    GemmArgs g{};
-    g.x = x;
-    g.wp = w.wp;
-    g.ws = w.ws;
-    g.wz = w.wz;
-    g.y = y;
-    g.M = M;
-    g.K = w.K;
-    g.N = w.N;
-    const GemvShape sh = gemv_shape(w, epi, M, ncu);
-    switch (w.form) {
-      case TGOHIP_FORM_F16: launch_gemv_form<TGOHIP_FORM_F16>(g, epi, sh, st); break;
-      case TGOHIP_FORM_I8: launch_gemv_form<TGOHIP_FORM_I8>(g, epi, sh, st); break;
-      case TGOHIP_FORM_I4_TGO: launch_gemv_form<TGOHIP_FORM_I4_TGO>(g, epi, sh, st); break;
-      case TGOHIP_FORM_I4_SYM: launch_gemv_form<TGOHIP_FORM_I4_SYM>(g, epi, sh, st); break;
-    }
-    TGOHIP_HIP(hipGetLastError());
-    return 0;
   }
-  const int MW = small_mw(w, M, ncu);
-  const int splits = choose_splits(M, w.N, w.K, MW, ncu);
-  const bool split_a = xk != XK_F16;  // f32 or an activation pair: hi + lo planes
   GemmArgs g{};
   g.x = x;
   g.xlo = xlo;
@@ -2037,27 +2054,39 @@ int gemm_enqueue(const PackedWeight& w, const void* x, int xk, int M, void* y, i
   g.M = M;
   g.K = w.K;
   g.N = w.N;
-  const int KS = w.K / 64;
-  g.ksteps_per_split = (KS + splits - 1) / splits;
-  if (splits > 1) {
-    if (!workspace || ws_bytes < (size_t)splits * split_plane_stride(M, w.N) * sizeof(float))
+  g.ksteps_per_split = r.ksteps_per_split;
+  if (r.splits > 1) {
+    if (!workspace || ws_bytes < (size_t)r.splits * split_plane_stride(M, w.N) * sizeof(float))
       return fail(TGOHIP_ESTATE, "linear: split-K workspace too small");
     g.part = workspace;
     g.pstride = split_plane_stride(M, w.N);
   }
-  const dim3 grid((unsigned)((w.N / 32 + 7) / 8), (unsigned)((M + MW - 1) / MW), (unsigned)splits);
-  if (MW == 32) {
-    if (split_a) launch_mw<32, true>(w.form, g, epi, grid, st);
-    else launch_mw<32, false>(w.form, g, epi, grid, st);
-  } else if (MW == 64) {
-    if (split_a) launch_mw<64, true>(w.form, g, epi, grid, st);
-    else launch_mw<64, false>(w.form, g, epi, grid, st);
+  if (r.kernel == TGOHIP_LINEAR_ROWS) {
+    launch_gemm_rows(w.form, g, xk, epi, r.cb, r.splits, st);
+  } else if (r.kernel == TGOHIP_LINEAR_GEMV) {
+    const GemvShape sh = gemv_shape(w, epi, M, ncu);
+    switch (w.form) {
+      case TGOHIP_FORM_F16: launch_gemv_form<TGOHIP_FORM_F16>(g, epi, sh, st); break;
+      case TGOHIP_FORM_I8: launch_gemv_form<TGOHIP_FORM_I8>(g, epi, sh, st); break;
+      case TGOHIP_FORM_I4_TGO: launch_gemv_form<TGOHIP_FORM_I4_TGO>(g, epi, sh, st); break;
+      case TGOHIP_FORM_I4_SYM: launch_gemv_form<TGOHIP_FORM_I4_SYM>(g, epi, sh, st); break;
+    }
   } else {
-    if (split_a) launch_mw<128, true>(w.form, g, epi, grid, st);
-    else launch_mw<128, false>(w.form, g, epi, grid, st);
+    const bool split_a = xk != XK_F16;  // f32 or an activation pair: hi + lo planes
+    const dim3 grid((unsigned)((w.N / 32 + 7) / 8), (unsigned)((M + r.mw - 1) / r.mw), (unsigned)r.splits);
+    if (r.mw == 32) {
+      if (split_a) launch_mw<32, true>(w.form, g, epi, grid, st);
+      else launch_mw<32, false>(w.form, g, epi, grid, st);
+    } else if (r.mw == 64) {
+      if (split_a) launch_mw<64, true>(w.form, g, epi, grid, st);
+      else launch_mw<64, false>(w.form, g, epi, grid, st);
+    } else {
+      if (split_a) launch_mw<128, true>(w.form, g, epi, grid, st);
+      else launch_mw<128, false>(w.form, g, epi, grid, st);
+    }
   }
-  if (defer) *defer = splits > 1 ? splits : 0;
-  if (splits > 1 && !defer) launch_reduce(g, epi, splits, st);
+  if (defer) *defer = r.splits > 1 ? r.splits : 0;
+  if (r.splits > 1 && !defer) launch_reduce(g, epi, r.splits, st);
   TGOHIP_HIP(hipGetLastError());
   return 0;
 }

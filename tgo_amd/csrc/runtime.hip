@@ -1482,6 +1482,20 @@ int tgohip_linear_workspace(tgohip_ctx* c, int handle, int x_dtype, int M, size_
   return 0;
 }
 
+int tgohip_linear_plan(int form, int K, int N, int x_dtype, int M, int epilogue, int ncu,
+                       tgohip_linear_plan_t* plan) {
+  const int rc = check_shape(form, K, N, "linear_plan");
+  if (rc) return rc;
+  if (M < 1 || ncu < 1 || epilogue < EPI_F32 || epilogue > EPI_SWIGLU_X2 || !plan)
+    return fail(TGOHIP_EINVAL, "linear_plan: M, ncu, epilogue and plan");
+  PackedWeight w;
+  w.form = form;
+  w.K = K;
+  w.N = N;
+  gemm_plan(w, M, ncu, xkind(x_dtype), epilogue, kScratchBytes, plan);
+  return 0;
+}
+
 int tgohip_dequant(tgohip_ctx* c, int handle, float* y) {
   PackedWeight* w = handle_of(c, handle);
   if (!w) return TGOHIP_EINVAL;
