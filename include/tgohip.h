@@ -254,19 +254,22 @@ int tgohip_linear(tgohip_ctx* ctx, int handle, const void* x, int x_dtype, int M
 /* tgohip_linear without allocating device memory. No counterpart in the
  * reference: it is for callers that cannot allocate (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). The caller
- * passes x and y; the split-K partials go to a static 64 MiB device array (one
- * per GPU, held until the process ends) instead of the context's workspace.
- * Same kernels and splits as tgohip_linear, so the same result. A call whose
- * partials need more than 64 MiB is refused (TGOHIP_EINVAL). Every call on a
- * GPU shares that GPU's array: calls that overlap on one GPU (two streams or
- * two contexts at once) race; calls in stream order do not. */
+ * passes x and y; the split-K partials, and the pair that f32 rows are split
+ * into, go to a static 64 MiB device array (one per GPU, held until the process
+ * ends) instead of the context's workspace. Same kernels and splits as
+ * tgohip_linear, so the same result; rows whose partials don't fit at once go
+ * in bands. A call for which tgohip_linear_workspace says more than 64 MiB is
+ * refused (TGOHIP_EINVAL). Every call on a GPU shares that GPU's array: calls
+ * that overlap on one GPU (two streams or two contexts at once) race, unless
+ * tgohip_linear_workspace says 0 for all but one of them; calls in stream order
+ * do not. */
 int tgohip_linear_noalloc(tgohip_ctx* ctx, int handle, const void* x, int x_dtype, int M,
                           void* y, int y_dtype);
-/* The split-K bytes by which tgohip_linear_noalloc takes or refuses a call over
- * M rows of a handle's weight with activations of x_dtype (TGOHIP_F16,
- * TGOHIP_F32 or TGOHIP_F16X2): it refuses calls above 64 MiB. What a call
- * writes there is at most this, or fits the array (few rows; f32 rows, which
- * may go in bands, with the same result). */
+/* Bytes of its array that tgohip_linear_noalloc asks for over M rows of a
+ * handle's weight with activations of x_dtype (TGOHIP_F16, TGOHIP_F32 or
+ * TGOHIP_F16X2): never less than the call writes; 0 when it leaves the array
+ * alone; above 64 MiB when it refuses the call. tgohip_linear_plan tells the
+ * bytes written (array_bytes) from those that decide (limit_bytes). */
 int tgohip_linear_workspace(tgohip_ctx* ctx, int handle, int x_dtype, int M, size_t* bytes);
 
 /* What a projection of M rows by a [K,N] weight of `form` runs on a GPU of

@@ -1,10 +1,10 @@
 """tgohip_linear_noalloc -- the linear whose split-K partials live in the library's
 static device workspace -- against tgohip_linear, through the C ABI: the same kernels and
 splits, so the outputs are equal to the bit. Two calls in a row, the second with fewer
-rows, so the second runs on the array the first left behind; every call here splits K
-(tgohip_linear_workspace says so), so both use the array; an empty batch launches nothing;
-a call needing more than the array holds is refused; and calls captured into a HIP graph
-replay to the same bits as eager calls."""
+rows, so the second runs on the array the first left behind (all but the int8 call at 48
+rows use it: there the row kernel needs no split); rows whose partials exceed the array go in
+bands; an empty batch launches nothing; a call beyond the limit is refused; and calls captured
+into a HIP graph replay to the same bits as eager calls."""
 import numpy as np
 import pytest
 
@@ -21,7 +21,8 @@ def weight(ctx, form, K, N, seed):
 @pytest.mark.parametrize("form,K,N,Ms,xf", [
     (tgo_amd.FORM_I4_SYM, 12288, 4096, (256, 40), tgo_amd.F16),   # pipelined kernel, 8 splits both
     (tgo_amd.FORM_I4_SYM, 12288, 4096, (1024, 512), tgo_amd.F16),  # 4 then 8 splits, 64 MiB each
-    (tgo_amd.FORM_I8, 4096, 6144, (64, 48), tgo_amd.F16),          # 8 splits both
+    (tgo_amd.FORM_I8, 4096, 6144, (64, 48), tgo_amd.F16),          # 8 splits, then none
+    (tgo_amd.FORM_I8, 4096, 6144, (96, 56), tgo_amd.F16),          # 8 splits both
     (tgo_amd.FORM_F16, 4096, 4096, (200, 33), tgo_amd.F32),       # gemm_kernel, 16 splits, f32 x
     (tgo_amd.FORM_I4_TGO, 4096, 12288, (130, 65), tgo_amd.F16),    # 3 then 4 splits
     (tgo_amd.FORM_I4_SYM, 4096, 4096, (128, 64), tgo_amd.F16X2),   # exact kernel, 8 splits both
@@ -33,6 +34,7 @@ def test_noalloc_linear_equals_linear(ctx, torch_gpu, form, K, N, Ms, xf):
         for M in Ms:
             print("no-alloc linear: form %d [%d,%d] M=%d" % (form, K, N, M), flush=True)
             assert ctx.linear_workspace(h, M, x_dtype=xf) > 0, "this call should split K"
+            assert (M, form) == (48, tgo_amd.FORM_I8) or tgo_amd.linear_plan(form, K, N, xf, M).array_bytes > 0
             g = torch.Generator(device="cuda").manual_seed(M)
             x = torch.randn(M, K, device="cuda", generator=g)
             if xf == tgo_amd.F16:
@@ -93,6 +95,26 @@ def test_noalloc_linear_refuses_beyond_its_workspace(ctx, torch_gpu):
             ctx.linear_noalloc(h, x, 2100, y)
         ctx.linear_noalloc(h, x, 2000, y)  # two planes of 32 MiB fit
         torch.cuda.synchronize()
+    finally:
+        ctx.weight_free(h)
+
+
+@pytest.mark.parametrize("form,K,N,M,xd,uses", [
+    (tgo_amd.FORM_I4_SYM, 1024, 24576, 1152, tgo_amd.F32, True),   # unsplit, but its pair is in the array
+    (tgo_amd.FORM_I4_SYM, 1024, 24576, 1152, tgo_amd.F16X2, False),
+    (tgo_amd.FORM_F16, 8192, 2048, 8, tgo_amd.F16X2, True),        # few rows, K in two shares
+    (tgo_amd.FORM_I8, 8192, 2048, 9, tgo_amd.F16, True),           # the row kernel splits f16 rows too
+    (tgo_amd.FORM_I8, 4096, 6144, 3, tgo_amd.F16, False),
+    (tgo_amd.FORM_F16, 1024, 65536, 150, tgo_amd.F16X2, True),
+])
+def test_workspace_query_covers_what_a_call_writes(ctx, torch_gpu, form, K, N, M, xd, uses):
+    """tgohip_linear_workspace is 0 only for a call that leaves the array alone."""
+    p = tgo_amd.linear_plan(form, K, N, xd, M)
+    assert (p.array_bytes > 0) == uses, (p.kernel, p.splits)
+    h = weight(ctx, form, K, N, 17)
+    try:
+        n = ctx.linear_workspace(h, M, x_dtype=xd)
+        assert n == max(p.array_bytes, p.limit_bytes)
     finally:
         ctx.weight_free(h)
 

@@ -615,11 +615,13 @@ class Context:
         return out
 
     def linear_noalloc(self, handle, x, M, y, x_dtype=F32, y_dtype=F32):
-        """linear with its split-K partials in the library's static workspace."""
+        """linear with what it writes on the way (split-K partials, the pair f32 rows are
+        split into) in the library's static array."""
         check(lib().tgohip_linear_noalloc(self.h, handle, ptr(x), x_dtype, M, ptr(y), y_dtype))
 
     def linear_workspace(self, handle, M, x_dtype=F32):
-        """Bytes of split-K partials a linear call over M rows uses (0: unsplit)."""
+        """Bytes of its static array that linear_noalloc asks for over M rows: at least what
+        the call writes (0: it leaves the array alone), above 64 MiB where it refuses it."""
         n = ctypes.c_size_t()
         check(lib().tgohip_linear_workspace(self.h, handle, x_dtype, M, ctypes.byref(n)))
         return n.value

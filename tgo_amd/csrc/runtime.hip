@@ -1478,7 +1478,9 @@ int tgohip_linear_workspace(tgohip_ctx* c, int handle, int x_dtype, int M, size_
   PackedWeight* w = handle_of(c, handle);
   if (!w) return TGOHIP_EINVAL;
   if (M < 0) return fail(TGOHIP_EINVAL, "linear_workspace: M is " + std::to_string(M));
-  *bytes = gemm_limit_bytes(*w, M, c->ncu, xkind(x_dtype));
+  // at least what the call writes, so that 0 says it leaves the array alone
+  *bytes = std::max(gemm_limit_bytes(*w, M, c->ncu, xkind(x_dtype)),
+                    gemm_call_bytes(*w, M, c->ncu, xkind(x_dtype), kScratchBytes));
   return 0;
 }
 
