@@ -1,8 +1,14 @@
 """The projections' dispatch rules (tgohip_linear_plan, host arithmetic) swept over forms,
 activations, widths and rows: every call the allocation-free linear takes fits its array."""
+import os
+import subprocess
+import sys
+
 import pytest
 
 import tgo_amd
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 ARRAY = 64 << 20
 WIDTHS = [(64, 128), (320, 6144), (1024, 6144), (1024, 65536), (1024, 151936), (1600, 34816), (1600, 49152),
@@ -34,3 +40,26 @@ def test_what_the_static_array_takes_fits_it(form, xd):
             assert p.splits == 1 or p.array_bytes > 0, at
             banded += whole > ARRAY
     assert banded or xd == tgo_amd.F16, "the widths reach calls whose planes go in bands"
+
+
+@pytest.mark.parametrize("most", [None, 1, 2, 4, 8])
+def test_max_splits_bounds_every_pipelined_call(most):
+    """TGOHIP_GEMM_MAX_SPLITS (read once per process) is the most split-K slices of the
+    pipelined kernel, in both arithmetics; unset, 8, and 16 with activation pairs."""
+    code = """
+import tgo_amd
+most = {}
+for form in range(4):
+    for xd in (tgo_amd.F32, tgo_amd.F16, tgo_amd.F16X2):
+        for K, N in [(1024, 6144), (1600, 4096), (4096, 4096), (4096, 6144), (12288, 4096), (25600, 5120)]:
+            for M in list(range(33, 200)) + [256, 353, 512, 1152, 1353]:
+                p = tgo_amd.linear_plan(form, K, N, xd, M)
+                if p.kernel == tgo_amd.LINEAR_PIPE:
+                    most[xd] = max(most.get(xd, 0), p.splits)
+print(most[tgo_amd.F32], most[tgo_amd.F16], most[tgo_amd.F16X2])
+"""
+    env = {k: v for k, v in os.environ.items() if not k.startswith("TGOHIP_")}
+    if most:
+        env["TGOHIP_GEMM_MAX_SPLITS"] = str(most)
+    out = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env=env, capture_output=True, text=True, check=True)
+    assert out.stdout.split() == ([str(most)] * 3 if most else ["16", "8", "16"])

@@ -1514,18 +1514,19 @@ static void launch_reduce(const GemmArgs& g, int epi, int splits, hipStream_t st
 // half the chip's slots (2 per CU); otherwise as many splits as fit in one
 // round of slots, keeping >= 8 k-steps per split.
 // slots: workgroups the chip holds at once.
-// TGOHIP_GEMM_MAX_SPLITS (1-8, default 8): the most split-K slices. At the
+// The most split-K slices: TGOHIP_GEMM_MAX_SPLITS (1-8) or, unset, 8, and 16
+// for the exact kernel's small grids (pipe_shape). At the
 // C4 decode step (128 rows) a cap of 4 (fewer partial planes for QKV and O)
 // or a rule keeping the planes' bytes below the weights' ran within the
 // run-to-run spread of 8 over 4 alternating pairs of 300 steps (10.64-10.91
 // against 10.62-10.65 ms); a cap of 2 was 5% slower.
-static int pipe_max_splits() {
+static int pipe_max_splits(bool ex) {
   static const int v = [] {
     const char* e = getenv("TGOHIP_GEMM_MAX_SPLITS");
-    const int n = e ? atoi(e) : 8;
-    return n >= 1 && n <= 8 ? n : 8;
+    const int n = e ? atoi(e) : 0;
+    return n >= 1 && n <= 8 ? n : 0;
   }();
-  return v;
+  return v ? v : ex ? 16 : 8;
 }
 
 // TGOHIP_GEMM_EX_SPLITS (0: the rule below): split-K count for the exact
@@ -1543,7 +1544,7 @@ static int choose_pipe_splits(int tiles, int KS, int slots) {
   if (tiles <= 0 || tiles >= slots / 2) return 1;  // the partial sums would cost more than the fill gains
   int s = slots / tiles;              // one round of workgroups
   while (s > 1 && KS / s < 8) s--;
-  return std::max(1, std::min(s, pipe_max_splits()));
+  return std::max(1, std::min(s, pipe_max_splits(false)));
 }
 
 // Row-tile height and split-K of the pipelined kernel. Up to 384 rows, 64-row
@@ -1599,7 +1600,9 @@ static void pipe_shape(const PackedWeight& w, int M, int ncu, int& mw, int& nw, 
   // int4 at 48 rows 8 -> 16 splits 28.5 -> 22.1 us, [1600, 4096] at 96 rows 3 -> 4
   // splits 17.6 -> 14.5 (without the reduction). With f16 operands, whose
   // k-steps are shorter, 16 splits cost [12288, 4096] 21.0 -> 22.4 with it.
-  while (ex && splits > 1 && splits < 16 && tiles * (splits + 1) <= ncu && (w.K / 64) / (splits + 1) >= 6) splits++;
+  if (ex) splits = std::min(splits, pipe_max_splits(true));
+  while (ex && splits > 1 && splits < pipe_max_splits(true) && tiles * (splits + 1) <= ncu && (w.K / 64) / (splits + 1) >= 6)
+    splits++;
   if (ex && pipe_ex_splits() > 0) {
     splits = pipe_ex_splits();
     while (splits > 1 && (w.K / 64) / splits < 8) splits--;
