@@ -63,3 +63,24 @@ print(most[tgo_amd.F32], most[tgo_amd.F16], most[tgo_amd.F16X2])
         env["TGOHIP_GEMM_MAX_SPLITS"] = str(most)
     out = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env=env, capture_output=True, text=True, check=True)
     assert out.stdout.split() == ([str(most)] * 3 if most else ["16", "8", "16"])
+
+
+@pytest.mark.parametrize("form", [0, 1, 2, 3])
+def test_the_row_kernel_gets_only_calls_that_it_has(form):
+    """It stores a SwiGLU (gate and up side by side: two column blocks a workgroup) as f16 or as
+    a pair, not as f32, and pairs column blocks over more than 32 rows for f16 weights with f16
+    rows or pairs only. Every combination of activation and epilogue that a call may have."""
+    rows = 0
+    for xd in (tgo_amd.F32, tgo_amd.F16, tgo_amd.F16X2):
+        for epi in ((0, 1, 2, 5) if xd == tgo_amd.F16X2 else (0, 1, 2, 3, 4)):
+            for K, N in WIDTHS:
+                for M in ROWS:
+                    p = tgo_amd.linear_plan(form, K, N, xd, M, epi)
+                    if p.kernel != tgo_amd.LINEAR_ROWS:
+                        continue
+                    rows += 1
+                    at = (form, K, N, xd, M, epi, p.column_blocks)
+                    assert epi != 4, at
+                    assert p.column_blocks == 2 or epi not in (3, 5), at
+                    assert p.column_blocks == 1 or M <= 32 or (form == tgo_amd.FORM_F16 and xd != tgo_amd.F32), at
+    assert rows > 1000

@@ -1817,6 +1817,9 @@ struct RowsShape {
 static RowsShape rows_shape(const PackedWeight& w, int xk, int M, int epi, int ncu) {
   const bool sw = epi == EPI_SWIGLU_F16 || epi == EPI_SWIGLU_X2;
   RowsShape r{0, 1};
+  // gemm_rows_kernel stores a SwiGLU as f16 or a pair, and over two row blocks of
+  // f32 rows it takes one column block, where a SwiGLU needs two
+  if (epi == EPI_SWIGLU_F32 || (sw && xk == XK_F32 && M > 32)) return r;
   const int KS = w.K / 64, mt = M > 32 ? (M + 63) / 64 : 1;
   int cb = sw ? 2 : 1;
   if (w.form == TGOHIP_FORM_F16 && xk != XK_F32 && M > 32 && w.N / 32 * mt > ncu && (w.N / 32 + 1) / 2 * mt <= ncu) cb = 2;
@@ -2065,7 +2068,7 @@ int gemm_enqueue(const PackedWeight& w, const void* x, int xk, int M, void* y, i
     g.pstride = split_plane_stride(M, w.N);
   }
   if (r.kernel == TGOHIP_LINEAR_ROWS) {
-    launch_gemm_rows(w.form, g, xk, epi, r.cb, r.splits, st);
+    if (const int rc = launch_gemm_rows(w.form, g, xk, epi, r.cb, r.splits, st)) return rc;
   } else if (r.kernel == TGOHIP_LINEAR_GEMV) {
     const GemvShape sh = gemv_shape(w, epi, M, ncu);
     switch (w.form) {

@@ -431,25 +431,29 @@ static void launch_rows_cb(const GemmArgs& g, int epi, int splits, hipStream_t s
 }
 
 template <int FORM>
-static void launch_rows_form(const GemmArgs& g, int xk, int epi, int cb, int splits, hipStream_t st) {
+static int launch_rows_form(const GemmArgs& g, int xk, int epi, int cb, int splits, hipStream_t st) {
 #define ROWS(XK)                                                                    \
   if (g.M <= 32 && cb == 1) launch_rows_cb<FORM, XK, 1, 1>(g, epi, splits, st);     \
   else if (g.M <= 32) launch_rows_cb<FORM, XK, 1, 2>(g, epi, splits, st);           \
   else if (cb == 1) launch_rows_cb<FORM, XK, 2, 1>(g, epi, splits, st);             \
   else if constexpr (FORM == TGOHIP_FORM_F16 && XK != XK_F32)                       \
-    launch_rows_cb<FORM, XK, 2, 2>(g, epi, splits, st)
+    launch_rows_cb<FORM, XK, 2, 2>(g, epi, splits, st);                             \
+  else return fail(TGOHIP_ESTATE, "linear: the row kernel takes no pair of column blocks here")
   if (xk == XK_F32) { ROWS(XK_F32); }
   else if (xk == XK_X2) { ROWS(XK_X2); }
   else { ROWS(XK_F16); }
 #undef ROWS
+  return 0;
 }
 
-void launch_gemm_rows(int form, const GemmArgs& g, int xk, int epi, int cb, int splits, hipStream_t st) {
+int launch_gemm_rows(int form, const GemmArgs& g, int xk, int epi, int cb, int splits, hipStream_t st) {
+  if (epi == EPI_SWIGLU_F32 || (cb == 1 && (epi == EPI_SWIGLU_F16 || epi == EPI_SWIGLU_X2)))
+    return fail(TGOHIP_ESTATE, "linear: the row kernel has no such SwiGLU store");
   switch (form) {
-    case TGOHIP_FORM_F16: launch_rows_form<TGOHIP_FORM_F16>(g, xk, epi, cb, splits, st); break;
-    case TGOHIP_FORM_I8: launch_rows_form<TGOHIP_FORM_I8>(g, xk, epi, cb, splits, st); break;
-    case TGOHIP_FORM_I4_TGO: launch_rows_form<TGOHIP_FORM_I4_TGO>(g, xk, epi, cb, splits, st); break;
-    default: launch_rows_form<TGOHIP_FORM_I4_SYM>(g, xk, epi, cb, splits, st); break;
+    case TGOHIP_FORM_F16: return launch_rows_form<TGOHIP_FORM_F16>(g, xk, epi, cb, splits, st);
+    case TGOHIP_FORM_I8: return launch_rows_form<TGOHIP_FORM_I8>(g, xk, epi, cb, splits, st);
+    case TGOHIP_FORM_I4_TGO: return launch_rows_form<TGOHIP_FORM_I4_TGO>(g, xk, epi, cb, splits, st);
+    default: return launch_rows_form<TGOHIP_FORM_I4_SYM>(g, xk, epi, cb, splits, st);
   }
 }
 

@@ -347,6 +347,6 @@ constexpr size_t kRowsPlaneBytes = (size_t)64 << 20;  // most bytes of its split
 // Whether M f32 or pair rows over `ksteps` k-steps fit a CU's LDS beside the
 // waves' sums.
 bool rows_staged(int M, int ksteps);
-void launch_gemm_rows(int form, const GemmArgs& g, int xk, int epi, int cb, int splits, hipStream_t st);
+int launch_gemm_rows(int form, const GemmArgs& g, int xk, int epi, int cb, int splits, hipStream_t st);
 
 }  // namespace tgohip
