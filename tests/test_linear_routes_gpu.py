@@ -75,8 +75,9 @@ def test_linear_over_any_whole_k_step(ctx, torch_gpu, form, K, N, M, xk):
 ])
 def test_linear_over_few_rows(ctx, torch_gpu, form, K, N, M, xk):
     """The row kernel at the edges of its launches: 1 to 16 rows staged in LDS (hi and lo
-    packed into one MFMA operand), 17 to 32 and 33 up from L2, k-steps that do not deal
-    evenly over the waves, shares of K, column blocks past the last whole round."""
+    packed into one MFMA operand), 17 up turned in LDS (up to 32 rows at one k-step a wave: from
+    L2), k-steps that do not deal evenly over the waves, shares of K, column blocks past the last
+    whole round."""
     check(torch_gpu, ctx, form, K, N, M, xk, 11 + K + M)
 
 
@@ -87,6 +88,7 @@ def test_linear_over_few_rows(ctx, torch_gpu, form, K, N, M, xk):
     (1088, 8192, 128),  # 17 k-steps over 8 waves, the pair of blocks at its largest
     (576, 128, 32), (512, 128, 33),  # just past and at one k-step a wave, one and two row blocks
     (4096, 2048, 48),   # split K, whole lines of every wave
+    (4096, 4224, 24),   # eight k-steps a wave through one row block's part of LDS
 ])
 def test_linear_turns_its_rows_in_lds(ctx, torch_gpu, form, K, N, M, xk):
     check(torch_gpu, ctx, form, K, N, M, xk, 11 + K + M)

@@ -104,7 +104,15 @@ __global__ __launch_bounds__(64 * W, W == 16 || (MB * CB == 1 && FORM != TGOHIP_
       }
     }
   };
-  // Only this wave reads what it writes here, and its LDS operations stay in order.
+  // Only this wave reads what it writes here, in its other lanes, and the hardware
+  // keeps a wave's LDS operations in order. The compiler sees each lane's own
+  // addresses, which hardly ever meet: turn0 (zero, but unknown to it) is in the
+  // reads' addresses, so that it cannot tell them from the writes' and keeps the
+  // order too. (A wave barrier or an LDS fence on both sides of the writes orders
+  // the global loads as well: int8 and symmetric int4 pairs then spill 13 to 55
+  // VGPRs.)
+  int turn0 = 0;
+  if constexpr (TURN) asm volatile("" : "+v"(turn0));
   auto store_turn = [&] {
     if constexpr (TURN) {
 #pragma unroll
@@ -157,7 +165,7 @@ __global__ __launch_bounds__(64 * W, W == 16 || (MB * CB == 1 && FORM != TGOHIP_
     } else if constexpr (TURN) {
 #pragma unroll
       for (int mb = 0; mb < MB; mb++) {
-        const half_t* const src = turn + (mb * 32 + c32) * 64 + 8 * rows_chunk(c32, 2 * j + h);
+        const half_t* const src = turn + turn0 + (mb * 32 + c32) * 64 + 8 * rows_chunk(c32, 2 * j + h);
         ah[mb] = *(const half8_t*)src;
         if constexpr (AP == 2) al[mb] = *(const half8_t*)(src + MB * 2048);
       }
