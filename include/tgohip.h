@@ -222,6 +222,17 @@ int tgohip_paged_attention_replay(tgohip_ctx* ctx, const void* q, int q_dtype, i
                                   const uint32_t* pages, int max_pages, int block, float scale,
                                   void* out, int out_dtype, int iters);
 
+/* How such a launch is decomposed, from its host arguments alone (no device, no
+ * counterpart in the reference): work items, parts of split contexts, and the
+ * most positions of an item that takes up to 16 query rows and of one that takes
+ * more. */
+typedef struct {
+  int32_t items, parts, longest_decode, longest_prefill;
+} tgohip_attention_plan_t;
+int tgohip_attention_plan(int T, int H, int H_kv, int capacity, int B, const uint32_t* lengths,
+                          const uint32_t* extents, const uint32_t* pages, int max_pages, int block,
+                          int q_dtype, tgohip_attention_plan_t* plan);
+
 /* Greedy selection over device logits [B,V] f32: ids[b] (device int32) is the
  * first index of the strict maximum of row b, the argmax of
  * sample/stages.go:196-206 (a NaN is never taken after index 0; NaN at index 0

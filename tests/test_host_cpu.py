@@ -780,3 +780,27 @@ def test_oracle_scheduler_known_answers():
     s.finish(0)
     assert s.admit([1, 2, 3]) == 0
     assert s.evict() == 0 and s.evict() == 1 and s.evict() == -1
+
+
+# ---- the attention launch's decomposition ---------------------------------------
+
+@pytest.mark.parametrize("extent", [1, 4, 5, 16, 64, 100, 512])
+@pytest.mark.parametrize("length", [512, 2048, 2049, 2100, 2560, 2561, 3000, 3072, 4096, 4097, 5000, 8192])
+def test_a_context_goes_into_few_equal_parts_of_at_most_2048_positions(length, extent):
+    """In a launch of one sequence the longest item is the launch's time: no item is longer than
+    the full 2048-position parts of prefill rows would be (parts of up to 3072 made 64 rows at
+    position 3070 take 94 us for 68), and parts of one context differ by less than a tile."""
+    H, Hkv, block = 32, 8, 16
+    pages = np.arange(-(-length // block), dtype=np.uint32)
+    p = tgo_amd.attention_plan(extent, H, Hkv, len(pages) * block, [length], [extent], pages, len(pages), block)
+    rows = extent * (H // Hkv)
+    longest = p.longest_decode if rows <= 16 else p.longest_prefill
+    assert (p.longest_prefill == 0) == (rows <= 16) and (p.longest_decode == 0) == (rows > 16)
+    assert longest <= 2048
+    # a row tile (32 tokens of 4 query heads) sees the positions up to its last token's
+    seen = [length] if rows <= 16 else [length - extent + min(extent, t + 32) for t in range(0, extent, 32)]
+    parts = [-(-n // 2048) for n in seen]
+    even = [n if c == 1 else -(-(-(-n // c)) // 64) * 64 for n, c in zip(seen, parts)]  # whole tiles
+    assert longest == max(even)
+    assert p.parts == Hkv * sum(c for c in parts if c > 1)
+    assert p.items == Hkv * sum(parts)

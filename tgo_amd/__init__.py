@@ -49,6 +49,10 @@ class LinearPlan(ctypes.Structure):
         (n, ctypes.c_size_t) for n in ("array_bytes", "limit_bytes")]
 
 
+class AttentionPlan(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int32) for n in ("items", "parts", "longest_decode", "longest_prefill")]
+
+
 class Timings(ctypes.Structure):
     _fields_ = [("submit_ms", ctypes.c_double), ("device_ms", ctypes.c_double),
                 ("readback_ms", ctypes.c_double)]
@@ -88,6 +92,7 @@ def lib():
         "tgohip_step": (I, [P, ctypes.POINTER(BatchStepC), P, P, ctypes.POINTER(Timings)]),
         "tgohip_paged_attention": (I, [P, P, I, I, I, I, I, P, P, I, I, P, P, P, I, I, F, P, I]),
         "tgohip_paged_attention_replay": (I, [P, P, I, I, I, I, P, P, I, I, P, P, P, I, I, F, P, I, I]),
+        "tgohip_attention_plan": (I, [I, I, I, I, I, P, P, P, I, I, I, ctypes.POINTER(AttentionPlan)]),
         "tgohip_weight_upload": (I, [P, I, I, I, P, P, P, P]),
         "tgohip_weight_synth": (I, [P, I, I, I, U64, U64, D, P]),
         "tgohip_weight_free": (I, [P, I]),
@@ -245,6 +250,15 @@ def linear_plan(form, K, N, x_dtype, M, epilogue=0, ncu=256):
     """What a projection runs (LinearPlan), by the library's dispatch rules alone: no GPU."""
     p = LinearPlan()
     check(lib().tgohip_linear_plan(form, K, N, x_dtype, M, epilogue, ncu, ctypes.byref(p)))
+    return p
+
+
+def attention_plan(T, H, Hkv, capacity, lengths, extents, pages, max_pages, block, q_dtype=F32):
+    """How a paged_attention launch is decomposed (AttentionPlan), without a GPU."""
+    lengths, extents, pages = u32(lengths), u32(extents), u32(pages)
+    p = AttentionPlan()
+    check(lib().tgohip_attention_plan(T, H, Hkv, capacity, len(lengths), ptr(lengths), ptr(extents), ptr(pages),
+                                      max_pages, block, q_dtype, ctypes.byref(p)))
     return p
 
 

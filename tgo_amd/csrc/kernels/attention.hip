@@ -863,12 +863,20 @@ int attn_build_plan(int T, int B, const uint32_t* lengths, const uint32_t* exten
   // Most positions per part of a context-split item (multiples of the 64-position
   // tile). Decode-style items stream, and long parts amortize a workgroup's start
   // (page staging, first loads) and merge; prefill-style items write 64 KiB of
-  // sums per part. Equal parts keep the launch's longest item short. Measured,
-  // equal parts, decode / prefill 2560 / 2048, 2560 / 3072, 2560 / 4096, 2048 /
-  // 2048 (us): 128 decodes 198.5, 198.3, 198.5, 195.3; 8 chunks of 256 beside 56
-  // decodes 199.7, 193.4, 241.5, 197.6; four chunks of 512, f16 q, 122.2, 120.7,
-  // 114.5, 122.0; with full parts and a remainder at 2560 / 2048: 201.1, 197.7,
-  // 126.0. Both depend only
+  // sums per part. In a launch of few items the longest one is what it takes; in
+  // one that fills the chip more parts cost their starts and merges. Kernel times,
+  // us, 32 heads over 8, most positions 2048 for both, in equal parts, against
+  // decode 2560 and prefill 2048 in full parts and a remainder:
+  //   prefill   64 rows at position 3070, f32 q 55 : 68, f16 q 42 : 50; 512 rows
+  //             f32 q 66 : 75; 8 chunks of 256 beside 56 decodes 193 : 197; four
+  //             chunks of 512 f16 q 117 : 121; but 1024 rows at 2100 83 : 77
+  //   decode    1 sequence of 2500 positions 26 : 42, 8 of them 28 : 44, 16 uniform
+  //             to 4096 41 : 48; but 32 of 2500 60 : 53, 64 116 : 107, 128 223 :
+  //             211, 128 lognormal 139 : 133
+  // Prefill parts of up to 3072 made 1024 rows at 2100 74 and the four chunks 115,
+  // but 64 rows at 3070 94 (f16 q 70), 512 rows 96: slower than full parts of 2048
+  // wherever few items run.
+  // Both depend only
   // on the sequence itself, so a mixed launch decomposes every sequence as it
   // would alone. TGOHIP_ATTN_SPLIT / TGOHIP_ATTN_PSPLIT override them.
   // An override is capped so that a part's page-16 table always fits the
@@ -886,6 +894,7 @@ int attn_build_plan(int T, int B, const uint32_t* lengths, const uint32_t* exten
   }();
   // Positions per part when `len` go into `parts`: equal parts of whole tiles,
   // not full ones and a remainder, so that the longest item of a launch is short.
+  // (A shared prefix and the suffixes after one keep full parts and a remainder.)
   auto even_part = [](int len, int parts) {
     return ((len + parts - 1) / parts + kAttnTile - 1) / kAttnTile * kAttnTile;
   };

@@ -1337,6 +1337,25 @@ int tgohip_paged_attention(tgohip_ctx* c, const void* q, int q_dtype, int T, int
                       H_kv, max_pages, block, scale, c->stream);
 }
 
+int tgohip_attention_plan(int T, int H, int H_kv, int capacity, int B, const uint32_t* lengths,
+                          const uint32_t* extents, const uint32_t* pages, int max_pages, int block,
+                          int q_dtype, tgohip_attention_plan_t* out) {
+  if (T < 0 || B < 0 || capacity <= 0 || !out) return fail(TGOHIP_EINVAL, "attention_plan: T, B, capacity and plan");
+  AttnPlan plan;
+  const int rc = attn_build_plan(T, B, lengths, extents, pages, max_pages, block, capacity, H, H_kv, plan, 0,
+                                 q_dtype != TGOHIP_F16);
+  if (rc) return rc;
+  *out = tgohip_attention_plan_t{0, plan.parts, 0, 0};
+  for (const AttnItem& it : plan.items) {
+    const int mode = it.mode & kAttnModeMask;
+    if (mode == 2) continue;  // an empty slot of the launch order
+    out->items++;
+    int32_t& most = mode == 1 ? out->longest_prefill : out->longest_decode;
+    most = std::max(most, it.kv_hi - it.kv_lo);
+  }
+  return 0;
+}
+
 // Plans once and replays the launch `iters` times (benchmark helper): the
 // metadata stays resident so each replay is the kernels alone.
 int tgohip_paged_attention_replay(tgohip_ctx* c, const void* q, int q_dtype, int T, int H, int H_kv,
