@@ -158,6 +158,39 @@ def test_a_permuted_page_table_equals_a_contiguous_cache(ctx, torch_gpu):
     assert not np.array_equal(a, c)
 
 
+@pytest.mark.parametrize("max_pages", [64, 25000])
+def test_calls_back_to_back_read_their_own_metadata(ctx, torch_gpu, max_pages):
+    """Twelve calls over other lengths and tables, none waited for, with page tables that a kernel
+    reads (4 KB) and that the copy engine takes (1.6 MB): each call's output is its own, by the
+    same call made alone with the smallest table."""
+    import tgo_amd
+    torch = torch_gpu
+    rng = np.random.default_rng(21)
+    H, Hkv, block, B, calls = 8, 2, 16, 16, 12
+    cap = B * 40 * block
+    k = torch.from_numpy(rng.standard_normal((cap, Hkv, DH)).astype(np.float16)).cuda()
+    v = torch.from_numpy(rng.standard_normal((cap, Hkv, DH)).astype(np.float16)).cuda()
+    q = torch.from_numpy(rng.standard_normal((B, H, DH)).astype(np.float32)).cuda()
+    ones = np.ones(B, np.uint32)
+
+    def call(out, lengths, table, width):
+        t = np.zeros((B, width), np.uint32)
+        t[:, :40] = table
+        ctx.paged_attention(q, B, H, Hkv, k, v, cap, lengths, ones, t, width, block, 0.088, out)
+
+    inputs = [(rng.integers(1, 40 * block + 1, B), rng.permutation(B * 40).reshape(B, 40)) for _ in range(calls)]
+    outs = [torch.full((B, H, DH), float("nan"), device="cuda") for _ in range(calls)]
+    assert (B * max_pages * 4 > 3 << 19) == (max_pages == 25000)  # 1.5 MiB: where the engine begins
+    for out, (lengths, table) in zip(outs, inputs):
+        call(out, lengths, table, max_pages)
+    torch.cuda.synchronize()
+    for out, (lengths, table) in zip(outs, inputs):
+        alone = torch.full((B, H, DH), float("nan"), device="cuda")
+        call(alone, lengths, table, 40)
+        torch.cuda.synchronize()
+        assert torch.isfinite(alone).all() and torch.equal(out, alone)
+
+
 def test_decode_equals_prefill_last_row(ctx, torch_gpu):
     """nn/attention_test.go:364 / oracle attention_test.go:153: a decode of the last token
     agrees with the chunk's last row (different work decomposition -> tolerance)."""
