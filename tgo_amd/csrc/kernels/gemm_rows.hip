@@ -16,7 +16,7 @@
 namespace tgohip {
 
 // k-steps of weight fragments a wave keeps in flight, by what the registers
-// allow: 128 with 16 waves (staged) or one 32 x 32 block per wave, else 256.
+// allow: 128 with 16 waves (staged) or four waves per SIMD, else 256.
 template <int FORM, int CB, bool STG> constexpr int rows_depth() {
   if (FORM == TGOHIP_FORM_I4_TGO && CB == 2) return 1;
   if (STG && CB == 1 && (FORM == TGOHIP_FORM_F16 || FORM == TGOHIP_FORM_I4_SYM)) return 4;
@@ -53,8 +53,12 @@ __device__ __forceinline__ int rows_chunk(int r, int c) { return c ^ (r & 7); }
 // bound the launch: [1024, 4096] of f16 weights at 67 pair rows 10.0 -> 6.8 us,
 // [3072, 1024] 11.2 -> 8.5, [4096, 6144] at 20 rows 20.6 -> 14.4.
 // Neither (PACK, or one k-step per wave): operands from L2.
+// Two waves per SIMD where 128 registers are not enough: int8's f32 rows and
+// pairs in TURN too (at four, 22 of them went to memory in every k-step: [4096,
+// 6144] at 20 pair rows 15.8 us against 12.8). tgo's int4 staged over 16 waves,
+// which have 128 registers and no more, spills 9.
 template <int FORM, int XK, int MB, int CB, bool PACK, bool STG, int W, bool TURN>
-__global__ __launch_bounds__(64 * W, W == 16 || (MB * CB == 1 && FORM != TGOHIP_FORM_I4_TGO && !(FORM == TGOHIP_FORM_I8 && XK == XK_F32 && TURN)) ? 4 : 2) void gemm_rows_kernel(
+__global__ __launch_bounds__(64 * W, W == 16 || (MB * CB == 1 && FORM != TGOHIP_FORM_I4_TGO && !(FORM == TGOHIP_FORM_I8 && XK != XK_F16 && TURN)) ? 4 : 2) void gemm_rows_kernel(
     GemmArgs g, int epi) {
   constexpr bool EX = XK != XK_F16;                          // tgo's arithmetic
   constexpr bool FX = EX && FORM == TGOHIP_FORM_I4_SYM;      // factored group scales
