@@ -26,11 +26,11 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 
 // dst[i] = host[i] over n 16-byte words, read across PCIe: a call's metadata
-// (tens to a few hundred KB) in stream order, without a copy engine's transfer
+// (up to kFetchBytes in runtime.hip) in stream order, without a copy engine's transfer
 // and the signals around it. With four staging slots, so that the host plans
 // the next call meanwhile, back-to-back attention calls lost their 15-25 us gap:
 // 128 decodes 198 -> 182 us, 8 chunks beside 56 decodes 204 -> 187, four chunks
-// of 512 rows 125 -> 109 (one box).
+// of 512 rows 125 -> 109.
 __global__ __launch_bounds__(256) void fetch_kernel(const uint4* host, uint4* dst, size_t n) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i < n) dst[i] = host[i];

@@ -213,12 +213,10 @@ __global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs g) {
   gemm_epilogue<EPI, MB>(g, acc, m0, nbw0, nbv, h, c32, gridDim.z > 1, blockIdx.z);
 }
 
-// Pipelined variant for f16 activations at larger M (the prefill-sized
-// projections). B fragments (the weight stream) for k-step j are issued at
-// step j-2 into a register ring; A (128 rows x 64 k of f16
-// activations, mostly L2-resident) is issued at step j-1 and written to a
-// double-buffered LDS tile at the end of that step. Barriers order LDS only, so
-// loads stay in flight across them.
+// Pipelined variant for larger M (the prefill-sized projections): f16
+// activations or, with EX, activation pairs. B fragments (the weight stream) go
+// into a register ring three k-steps ahead (f16 weights two); A (64 or 128 rows
+// x 64 k, mostly L2-resident) goes to a four-stage LDS ring by DMA, three ahead.
 // ---- the pipelined kernel's B operand per form ------------------------------
 // The register part of one (column block, k-step) of B. For int8 and tgo's
 // int4 the per-k scales (and zeros) are the same for the 32 columns of a
@@ -348,9 +346,11 @@ __device__ __forceinline__ void pipe_bfrag_x(const PipeB<TGOHIP_FORM_I8>& r, int
 // tgo's f32 dequantize-then-dot up to f32 rounding order, with the lo.lo term
 // (2^-22 relative) dropped as in the three-MFMA form.
 // TAIL: K may leave one to three k-steps after its groups of four. The tail
-// costs the factored kernel 1% at [4096, 24576] over 1152 rows (394-397 us
-// without, 399-401 with: its registers go from 238 to 256), so that kernel is
-// built both ways; the others are as fast with it.
+// takes the factored kernel's registers from 238 to 256 and costs it 1% at
+// [4096, 24576] (three alternating pairs of runs, without : with, 395.6-396.7 :
+// 398.5-400.2 us over 1152 rows, 497-498 : 502 over 1353) and 3% at [4096, 6144]
+// (108 : 110-112), so that kernel is built both ways; the others are as fast
+// with it.
 template <int FORM, int EPI, int MW, int NW, int KQ = 1, bool EX = false, bool TAIL = true>
 __global__ __launch_bounds__((64 * NW * KQ), (8 / (NW * KQ))) void gemm_pipe_kernel(
     GemmArgs g, int tiles_n, int tiles, int colmajor, int xsplit, QKRopeArgs qa) {
@@ -478,11 +478,12 @@ __global__ __launch_bounds__((64 * NW * KQ), (8 / (NW * KQ))) void gemm_pipe_ker
   // k % 4, DMA'd in the middle of step k-3; B(k) in register slot k % 4,
   // loaded at the start of step k-3 (the slot of B(k-4), whose last read
   // was in step k-4; three steps ahead cut the M = 128 gate/up from 46 to
-  // 41 us). Each step reads the next step's first
+  // 41 us), with f16 weights of step k-2 (pipe_b_ahead). Each step reads the next step's first
   // fragments during its last substep, so the MFMAs run on across step
   // boundaries. One barrier per step, in its middle. Before it a wave waits
   // for its own DMA of stage k+1 (issued at step k-2: the vector memory
-  // operations issued since are B(k+2), stage k+2's DMA and B(k+3)) and for its
+  // operations issued since are B(k+2), stage k+2's DMA and B(k+3), or with f16
+  // weights B(k+1), the DMA and B(k+2): as many) and for its
   // LDS reads; past it, stage k+1 is visible to every wave, and every wave is
   // done reading stage k-1, which the DMA of stage k+3 issued right after the
   // barrier reuses. The barrier carries no memory fence: a fence would wait
@@ -793,10 +794,11 @@ __global__ __launch_bounds__((64 * NW * KQ), (8 / (NW * KQ))) void gemm_pipe_ker
   } else {
     // Each wave turns its sums through 8 KiB of the ring, 32 rows x 64 columns at
     // a time, so that it stores whole 16-byte pieces of a row instead of single
-    // words (64 stores a wave, 4.1 us of a 128-row projection's 14 to 35): [4096,
-    // 4096] of symmetric int4 at 128 pair rows, 8 splits, 17.6 -> 15.8 us, [12288,
-    // 4096] 35.4 -> 33.5, [4096, 24576] at 1152 rows 406 -> 399; f16 operands 21.3
-    // -> 17.9, 37.7 -> 34.5, 209 -> 205. Every wave is done reading the ring; with two k groups the other
+    // words (64 stores a wave). Whole calls over symmetric int4, single words :
+    // pieces, three alternating pairs of runs, us: pairs [4096, 4096] at 128 rows
+    // 25.4 : 23.8, [12288, 4096] 37.6 : 36.0, at 1152 rows 233 : 229, [4096, 24576]
+    // at 1152 409 : 403; f16 operands [4096, 12288] at 128 29.7 : 27.6, at 1024
+    // 98.6 : 96.5, [4096, 24576] at 1152 211 : 208. Every wave is done reading the ring; with two k groups the other
     // group has ended and this wave alone read its part of it.
     if constexpr (KQ == 1) __syncthreads();
     const int wst = NW == 8 ? wave >> 1 : wave;
@@ -1452,7 +1454,10 @@ static int choose_splits(int M, int N, int K, int MW, int ncu) {
 
 // gemm_kernel's row tile: 32, 64 or 128 rows by M; 32 for a batch of at most
 // 128 rows whose grid would not give every CU a workgroup (the C1 step, 67
-// rows over f16 weights: 3.05 -> 2.05 ms per step with two-k-step splits).
+// rows over f16 weights: 3.05 -> 2.05 ms per step with two-k-step splits; those
+// rows run gemm_rows_kernel since). What gemm_route leaves to it takes 32 rows, or
+// 128 for f16 operands over f16 weights and where the pipelined kernel's 32-bit
+// offsets don't reach (M K from 2^31); 64 only with TGOHIP_GEMM_PIPE_MIN raised.
 static int small_mw(const PackedWeight& w, int M, int ncu) {
   const int mw = M <= 32 ? 32 : (M <= 64 ? 64 : 128);
   const int col_tiles = (w.N / 32 + 7) / 8;
